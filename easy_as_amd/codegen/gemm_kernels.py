@@ -42,12 +42,12 @@ is 4-byte aligned; each matrix under 2 GiB):
   MFMAs overlap the DMA issue (one every two MFMAs) and the next stage's ks0
   fragment reads.
 
-Register body (any other case, including f32 inputs that MFMA consumes as f16):
-global -> registers -> LDS, BK = 64, double buffered; A loads use the widest
-vector (up to 16 bytes) that K's row alignment allows; B is transposed in
-registers (each thread loads an 8(k) x 8(n) block) so LDS holds B as [n][k];
-edge tiles and the K tail load element by element with zero fill straight into
-LDS.
+Register bodies (any other case, including f32 inputs that MFMA consumes as f16):
+global -> registers -> LDS in the DMA bodies' layouts, rounding on the way; 16-byte
+loads at any element alignment, with the ends of rows and buffers moved into place in
+registers.  Launches of at most 64 rows split K over the four waves of a 64-column
+group; others run 64 x 64, 128 x 64, 128 x 128 or 256 x 256 tiles, whichever the launch
+plan's cost rule picks.
 
 Tile order is XCD aware: workgroup w runs on XCD w % 8, so each XCD gets a
 contiguous range of tiles, grouped 4 tile-rows high for L2 reuse.
@@ -126,43 +126,58 @@ _TEMPLATE = r"""
 typedef eas_op_t eas_h8 __attribute__((ext_vector_type(8)));
 typedef eas_op_t eas_h4 __attribute__((ext_vector_type(4)));
 
-template <typename T> static __device__ __forceinline__ eas_h8 eas_load8(const T* p);
-template <> __device__ __forceinline__ eas_h8 eas_load8<eas_op_t>(const eas_op_t* p) { return *(const eas_h8*)p; }
-template <> __device__ __forceinline__ eas_h8 eas_load8<float>(const float* p) {
-  const eas_f32x4 lo = *(const eas_f32x4*)p, hi = *(const eas_f32x4*)(p + 4);
-  eas_h8 v;
-  v[0] = (eas_op_t)lo[0]; v[1] = (eas_op_t)lo[1]; v[2] = (eas_op_t)lo[2]; v[3] = (eas_op_t)lo[3];
-  v[4] = (eas_op_t)hi[0]; v[5] = (eas_op_t)hi[1]; v[6] = (eas_op_t)hi[2]; v[7] = (eas_op_t)hi[3];
-  return v;
+// The bodies that load through registers (operands the DMA cannot take) move 16-byte units of any
+// element alignment: global loads accept every alignment on this target, so rows of odd length and
+// fp32 operands load as wide as aligned ones.  A unit holds eas_unit<T>() elements of one row.
+typedef uint32_t eas_u32x4 __attribute__((ext_vector_type(4)));
+typedef eas_u32x4 eas_u32x4_any __attribute__((aligned(2), may_alias));
+template <typename T> constexpr int eas_unit() { return 16 / (int)sizeof(T); }
+template <typename T> static __device__ __forceinline__ eas_u32x4 eas_load_unit(const T* p) {
+  return *(const eas_u32x4_any*)p;
 }
-
-// elements per load for rows of `k` elements of T: the widest power of two up to 16 bytes dividing k
-template <typename T> constexpr int eas_row_vec(int k) {
-  int v = 16 / (int)sizeof(T);
-  while (v > 1 && k % v != 0) v /= 2;
-  return v;
+// threadIdx.x as a value of its own: the address arithmetic of the bodies sharing an entry is not
+// merged and kept in registers across their branches (with it merged, the entry spilled)
+static __device__ __forceinline__ int eas_tid() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
 }
-// 8 consecutive elements from rows whose alignment allows AL-element vector loads
-template <typename T, int AL> static __device__ __forceinline__ eas_h8 eas_load8_al(const T* p) {
-  if constexpr (AL >= 8 && sizeof(T) == 2) {
-    return *(const eas_h8*)p;
-  } else if constexpr (AL == 1) {
-    eas_h8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (eas_op_t)p[e];
-    return v;
+// the unit `bits` bits down (0 <= bits < 128), zeros from the top
+static __device__ __forceinline__ eas_u32x4 eas_unit_down(eas_u32x4 v, uint32_t bits) {
+  const uint32_t v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3];
+  const uint64_t lo = (uint64_t)v0 | ((uint64_t)v1 << 32), hi = (uint64_t)v2 | ((uint64_t)v3 << 32);
+  const uint32_t b = bits & 63u;
+  const uint64_t up = b ? hi << (64u - b) : 0ull;
+  const uint64_t l = bits >= 64u ? hi >> b : (lo >> b) | up, h = bits >= 64u ? 0ull : hi >> b;
+  return (eas_u32x4){(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
+}
+// a unit's elements, rounded to the operand type, into LDS
+template <typename T> static __device__ __forceinline__ void eas_store_unit(eas_op_t* dst, eas_u32x4 v) {
+  if constexpr (sizeof(T) == 4) {
+    const eas_f32x4 f = __builtin_bit_cast(eas_f32x4, v);
+    const float f0 = f[0], f1 = f[1], f2 = f[2], f3 = f[3];
+    *(eas_h4*)dst = (eas_h4){(eas_op_t)f0, (eas_op_t)f1, (eas_op_t)f2, (eas_op_t)f3};
   } else {
-    constexpr int W = AL > 8 ? 8 : AL;
-    typedef T vec_t __attribute__((ext_vector_type(W)));
-    eas_h8 v;
+    typedef T vec_t __attribute__((ext_vector_type(8)));
+    const vec_t x = __builtin_bit_cast(vec_t, v);
+    eas_h8 h;
 #pragma unroll
-    for (int e = 0; e < 8; e += W) {
-      const vec_t x = *(const vec_t*)(p + e);
-#pragma unroll
-      for (int i = 0; i < W; ++i) v[e + i] = (eas_op_t)x[i];
-    }
-    return v;
+    for (int e = 0; e < 8; ++e) h[e] = (eas_op_t)x[e];
+    *(eas_h8*)dst = h;
   }
+}
+// Units at the ends of the operands.  A row of A ends at K, which a unit may straddle; the last row
+// of B ends at column N, which is where the buffer may end (in the rows above it, elements past N
+// belong to the next row, and columns past N are never stored).  A straddling unit loads from
+// that many elements earlier (inside the operand for K >= 8 and ldb >= 8) and moves down after the
+// load.  Units wholly past K are zero in A and in B: either could hold a NaN or an infinity.
+// `lost`: how many elements of the unit at `at` lie past `end`, in [0, unit].
+template <typename T> static __device__ __forceinline__ int eas_unit_lost(int at, int end) {
+  constexpr int U = eas_unit<T>();
+  return at + U <= end ? 0 : at >= end ? U : at + U - end;
+}
+template <typename T> static __device__ __forceinline__ eas_u32x4 eas_unit_end(eas_u32x4 v, int lost) {
+  return lost >= eas_unit<T>() ? (eas_u32x4){} : eas_unit_down(v, (uint32_t)(lost * (int)sizeof(T) * 8));
 }
 
 template <typename CT, int K>
@@ -173,7 +188,7 @@ static __device__ __forceinline__ void eas_gemm_dma(const eas_op_t* __restrict__
   constexpr int STAGE_H = BM * BK;  // halves per operand per stage (16 KB)
   eas_op_t* As = smem;
   eas_op_t* Bs = smem + NSTAGE * STAGE_H;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = eas_tid(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const eas_rsrc ra = eas_make_rsrc(A, (uint32_t)M * (uint32_t)K * 2u);
@@ -893,7 +908,7 @@ static __device__ __forceinline__ void eas_gemm_skinny_dma(const eas_op_t* __res
   static_assert(4 * NST * STH * 2 <= 147456, "the rings fit the entry's LDS");
   constexpr int NBQ = NT / 16, CH = NT / 8;                     // B DMA instructions per stage, chunks per row
   constexpr int LOADS = NBQ + MT;                               // DMA instructions per stage
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = eas_tid(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kb = wave * KW, ke = min(K, kb + KW);
   const int nsteps = ke > kb ? (ke - kb + KS - 1) / KS : 0;
@@ -1002,175 +1017,357 @@ static __device__ __forceinline__ void eas_gemm_skinny_dma(const eas_op_t* __res
   }
 }
 
-// Skinny path for inputs the DMA cannot take (f32 or unaligned): one thread per (column, 4 MT rows)
-// of the 64 columns from n0.
+// Skinny path for inputs the DMA cannot take (f32, or rows of A or B not 16-byte aligned): 64 columns
+// from n0, the four waves split K as above, each moving its range global -> registers -> LDS, R
+// stages of 32 k in flight in registers.  A wave's LDS accesses run in order, so its private slot
+// needs no barrier.  Bound by the rows of B from HBM where the grid fills the chip, else by the latency of
+// a wave's chain of stages.  f16 16 x 14336 x 4097: 18.6 us, 6.3 TB/s; f32 16 x 14336 x 4096: 34.1 us,
+// 6.9 TB/s.  More stages in flight (4, 6) take AGPRs and moves between them: 20.3 and 20.8 us.
 template <typename AT, typename BT, typename CT, int K, int MT>
-static __device__ __forceinline__ void eas_gemm_skinny_simple(const AT* __restrict__ A, const BT* __restrict__ B,
-                                                              CT* __restrict__ C, int ldb, int M, int N, int n0) {
-  constexpr int R = 4 * MT;  // rows per thread: r0, r0 + 4, ...
-  const int tid = threadIdx.x, col = n0 + (tid & 63), r0 = tid >> 6;
-  if (col >= N) return;
-  float acc[R];
+static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict__ A, const BT* __restrict__ B,
+                                                            CT* __restrict__ C, int ldb, int M, int N, int n0,
+                                                            eas_op_t* smem) {
+  constexpr int KS = 32, MR = 16 * MT, NT = 64, NJ = NT / 16;
+  constexpr int KW = ((K + 4 * KS - 1) / (4 * KS)) * KS;  // k rows per wave
+  constexpr int UA = eas_unit<AT>(), UB = eas_unit<BT>();
+  constexpr int ACH = KS / UA, BCH = NT / UB;                  // units per row of A (within a stage) and of B
+  constexpr int NA = MR * ACH / 64, NB = KS * BCH / 64;        // units per lane and stage
+  constexpr int R = NA + NB <= 6 ? 2 : 1;                      // stages in flight
+  constexpr int STH = KS * NT + MR * KS;                       // halves: B [32][64], A [MR][32]
+  const int tid = eas_tid(), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kb = wave * KW, ke = min(K, kb + KW);
+  const int nsteps = ke > kb ? (ke - kb + KS - 1) / KS : 0;
+  eas_op_t* bs = smem + wave * STH;
+  eas_op_t* as = bs + KS * NT;
+  auto swz = [](int r) { return 2 * ((r >> 1) & 1) + 4 * ((r >> 3) & 1); };  // as the DMA path's, 128-byte rows
+  const AT* pa[NA];
+  const BT* pb[NB];
+  int la[NA], lb[NB];
 #pragma unroll
-  for (int i = 0; i < R; ++i) acc[i] = 0.0f;
-  for (int k = 0; k < K; ++k) {
-    const float b = (float)(eas_op_t)B[(size_t)k * ldb + col];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const int row = r0 + 4 * i;
-      const float a = row < M ? (float)(eas_op_t)A[(size_t)row * K + k] : 0.0f;
-      acc[i] = __builtin_fmaf(a, b, acc[i]);
-    }
+  for (int i = 0; i < NA; ++i) {
+    const int r = (64 / ACH) * i + lane / ACH, e = (lane % ACH) * UA;
+    pa[i] = A + (size_t)min(r, M - 1) * K + kb + e;
+    la[i] = r * KS + (((e >> 3) ^ ((r >> 2) & 3)) * 8) + (e & 7);
   }
+  const int be = (lane % BCH) * UB, bn = n0 + be < N ? n0 + be : 0;
 #pragma unroll
-  for (int i = 0; i < R; ++i)
-    if (r0 + 4 * i < M) C[(size_t)(r0 + 4 * i) * ldb + col] = (CT)acc[i];
+  for (int i = 0; i < NB; ++i) {
+    const int r = (64 / BCH) * i + lane / BCH;
+    pb[i] = B + (size_t)(kb + r) * ldb + bn;
+    lb[i] = r * NT + (((be >> 3) ^ swz(r)) * 8) + (be & 7);
+  }
+  // how much of a unit lies past the operand, in the stage that holds the last row of B
+  auto lost_a = [&](int t, int i) { return eas_unit_lost<AT>(kb + t * KS + (lane % ACH) * UA, K); };
+  auto lost_b = [&](int t, int i) {
+    const int k = kb + t * KS + (64 / BCH) * i + lane / BCH;
+    return k >= K ? UB : k == K - 1 ? eas_unit_lost<BT>(bn, N) : 0;
+  };
+  eas_u32x4 ra[R][NA], rb[R][NB];
+  auto load = [&](int t, eas_u32x4 (&xa)[NA], eas_u32x4 (&xb)[NB]) {
+    if (kb + (t + 1) * KS < K) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) xb[i] = eas_load_unit(pb[i] + (size_t)t * KS * ldb);
+#pragma unroll
+      for (int i = 0; i < NA; ++i) xa[i] = eas_load_unit(pa[i] + t * KS);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int lost = lost_b(t, i);
+        xb[i] = eas_load_unit(lost == UB ? B : pb[i] + (size_t)t * KS * ldb - lost);
+      }
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const int lost = lost_a(t, i);
+        xa[i] = eas_load_unit(lost == UA ? A : pa[i] + t * KS - lost);
+      }
+    }
+  };
+  const int fm = lane & 15;
+  const int fa = fm * KS + (((lane >> 4) ^ ((fm >> 2) & 3)) * 8);
+  int fb[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int g = lane >> 4, kq = lane & 15;
+    const int row = 8 * g + (kq >> 2), col = 16 * j + 4 * (kq & 3);
+    fb[j] = row * NT + ((col >> 3) ^ swz(row)) * 8 + (col & 7);
+  }
+  eas_f32x4 acc[MT][NJ];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[mt][j] = (eas_f32x4){};
+  auto step = [&](int t, eas_u32x4 (&xa)[NA], eas_u32x4 (&xb)[NB]) {
+    if (kb + (t + 1) * KS >= K) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) xb[i] = eas_unit_end<BT>(xb[i], lost_b(t, i));
+#pragma unroll
+      for (int i = 0; i < NA; ++i) xa[i] = eas_unit_end<AT>(xa[i], lost_a(t, i));
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) eas_store_unit<BT>(bs + lb[i], xb[i]);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) eas_store_unit<AT>(as + la[i], xa[i]);
+    if (t + R < nsteps) load(t + R, xa, xb);
+    eas_h8 a[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) a[mt] = *(const eas_h8*)(as + mt * 16 * KS + fa);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const eas_h4t lo = EAS_DS_TR16((EAS_LDS eas_h4t*)(bs + fb[j]));
+      const eas_h4t hi = EAS_DS_TR16((EAS_LDS eas_h4t*)(bs + fb[j] + 4 * NT));
+      const eas_h4 l4 = __builtin_bit_cast(eas_h4, lo), h4 = __builtin_bit_cast(eas_h4, hi);
+      const eas_h8 b = (eas_h8){l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt][j] = EAS_MFMA16(a[mt], b, acc[mt][j], 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < R; ++p)
+    if (p < nsteps) load(p, ra[p], rb[p]);
+  for (int t = 0; t < nsteps; t += R)
+#pragma unroll
+    for (int p = 0; p < R; ++p)
+      if (t + p < nsteps) step(t + p, ra[p], rb[p]);
+  // every load has been used: said here, so that the compiler does not take them for pending in the
+  // entry's other bodies and wait between their DMA loads (decode launches ran 3-8 us longer)
+  __builtin_amdgcn_s_waitcnt(EAS_WAITVM(0));
+  // the waves' partial sums meet in LDS, as in the DMA path
+  float* red = (float*)smem;  // [4 waves][MR][NT]
+  static_assert(4 * MR * NT * 4 <= 147456, "the reduction fits the LDS");
+  __syncthreads();
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[(wave * MR + 16 * mt + 4 * (lane >> 4) + r) * NT + 16 * j + (lane & 15)] = acc[mt][j][r];
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < MR * NT / 256; ++e) {
+    const int idx = tid + 256 * e, row = idx / NT, col = idx % NT;
+    const float sum = (red[row * NT + col] + red[(MR + row) * NT + col]) +
+                      (red[(2 * MR + row) * NT + col] + red[(3 * MR + row) * NT + col]);
+    if (row < M && n0 + col < N) C[(size_t)row * ldb + n0 + col] = (CT)sum;
+  }
+  __syncthreads();  // the sums are read: a second call on the next columns may refill the LDS
 }
 
-template <typename AT, typename BT, typename CT, int K>
+// Tile body for operands the DMA cannot take (f32, odd K, odd ldb, odd addresses): BM x BN tiles, 4 waves
+// of BM/2 x BN/2.  Each wave moves its share of a stage global -> registers -> LDS (two slots), rounding
+// to the operand type on the way, in the DMA bodies' LDS layouts, so B is transposed by
+// ds_read_b64_tr_b16 and costs no VALU.  256 x 256: BK = 32 on 32x32x16 MFMAs; smaller
+// tiles: BK = 64 on 16x16x32, so that a row's stage is 128 bytes (256 of f32) and a row that starts at
+// an odd address straddles one more line in two, not in one.
+//
+// One barrier per stage, in its middle.  Before it: the MFMAs of the first k half, the reads of
+// the second half's fragments, the stores of stage kt+1 into the other slot (last read before the
+// previous barrier) and the loads of stage kt+2 into the registers this frees.  After it: the MFMAs
+// of the second half and the reads of stage kt+1's first fragments.A second stage
+// in flight needs registers past 256, which cost moves from and to AGPRs: 1024 x 2048 x 2048 f32 on 128 x 64
+// tiles 27.1 us with one stage, 36.5 with two.  Bound by the rate a CU takes lines from L2: a 16-byte
+// load off a 16-byte boundary takes two passes (59 B/ns against 117 aligned in a read loop), so a 128 x 128 x
+// 64 stage of odd rows is about 0.55 us of loads for 0.24 us of MFMAs; 1531 x 2047 x 1023 f16 runs 16.6 us
+// (with the element-wise body this replaces 125.8), 4095^3 140 us = 978 TFLOP/s.
+template <typename AT, typename BT, typename CT, int K, int BM, int BN>
 static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, const BT* __restrict__ B,
                                                      CT* __restrict__ C, int ldb, int M, int N, int m0, int n0,
                                                      eas_op_t* smem) {
-  constexpr int BM = 256, BN = 256, BK = 64, WN = 2, NTHREADS = 256, TI = 4, TJ = 4;
-  constexpr int PITCH = BK + 8, KC = BK / 8, A_IT = BM * BK / 8 / NTHREADS, NBLK = BK * BN / 64;
-  constexpr int B_IT = (NBLK + NTHREADS - 1) / NTHREADS;
-  eas_op_t* As0 = smem;  // [2][BM * PITCH]
-  eas_op_t* Bs0 = smem + 2 * BM * PITCH;  // [2][BN * PITCH]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  // A rows (length K, compile time) load A_AL elements per vector; B rows need 16-byte vectors
-  // (ldb a multiple of 16 bytes, aligned base).  Anything else takes the masked element path.
-  constexpr int A_AL = eas_row_vec<AT>(K);
-  const bool mn_full = (m0 + BM <= M) && (n0 + BN <= N) && (ldb % (16 / (int)sizeof(BT)) == 0) &&
-                       ((uint64_t)B % 16 == 0) && ((uint64_t)A % (A_AL * sizeof(AT)) == 0);
-
-  eas_h8 ra[A_IT], rb[B_IT][8];
-  auto gload_fast = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < A_IT; ++i) {
-      const int c = tid + NTHREADS * i, row = c / KC, kc = c % KC;
-      ra[i] = eas_load8_al<AT, A_AL>(A + (size_t)(m0 + row) * K + k0 + kc * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < B_IT; ++i) {
-      const int blk = tid + NTHREADS * i, kg = blk % KC, nc = blk / KC;
-      if (NBLK % NTHREADS != 0 && blk >= NBLK) break;
-#pragma unroll
-      for (int r = 0; r < 8; ++r) rb[i][r] = eas_load8<BT>(B + (size_t)(k0 + kg * 8 + r) * ldb + n0 + nc * 8);
-    }
+  constexpr int MI = BM == 256 ? 32 : 16, BK = BM == 256 ? 32 : 64, KT = (K + BK - 1) / BK;
+  constexpr int TI = BM / 2 / MI, TJ = BN / 2 / MI;
+  constexpr int UA = eas_unit<AT>(), UB = eas_unit<BT>(), ACH = BK / UA, BCH = BN / UB;
+  constexpr int NA = BM * ACH / 256, NB = BK * BCH / 256;  // units per lane and stage
+  constexpr int STAGE_A = BM * BK, STAGE_B = BK * BN;
+  eas_op_t* As = smem;
+  eas_op_t* Bs = smem + 2 * STAGE_A;
+  static_assert(2 * (STAGE_A + STAGE_B) * 2 <= 147456, "the slots fit the entry's LDS");
+  const int tid = eas_tid(), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // 16-byte chunks of A's row r at chunk ^ asw(r), of B's row r at chunk ^ bsw(r): the DMA bodies'
+  // masks, and for 128-byte rows of A the fp32 entries'
+  auto asw = [](int r) { return BK == 64 ? (r >> 1) & 7 : (r >> 2) & 3; };
+  auto bsw = [](int r) {
+    return BN == 64 ? 2 * ((r >> 1) & 1) + 4 * ((r >> 3) & 1) : (4 * (r & 3)) ^ (2 * ((r >> 3) & 1));
   };
-  auto sstore_regs = [&](int buf) {
-    eas_op_t* As = As0 + buf * BM * PITCH;
-    eas_op_t* Bs = Bs0 + buf * BN * PITCH;
+  const AT* pa[NA];
+  const BT* pb[NB];
+  int la[NA], lb[NB];
+  const int ae = (tid % ACH) * UA;
 #pragma unroll
-    for (int i = 0; i < A_IT; ++i) {
-      const int c = tid + NTHREADS * i, row = c / KC, kc = c % KC;
-      *(eas_h8*)(&As[row * PITCH + kc * 8]) = ra[i];
-    }
+  for (int i = 0; i < NA; ++i) {
+    const int r = (256 / ACH) * i + tid / ACH;
+    pa[i] = A + (size_t)min(m0 + r, M - 1) * K + ae;
+    la[i] = r * BK + (((ae >> 3) ^ asw(r)) * 8) + (ae & 7);
+  }
+  const int be = (tid % BCH) * UB, bn = n0 + be < N ? n0 + be : 0;
 #pragma unroll
-    for (int i = 0; i < B_IT; ++i) {
-      const int blk = tid + NTHREADS * i, kg = blk % KC, nc = blk / KC;
-      if (NBLK % NTHREADS != 0 && blk >= NBLK) break;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        eas_h8 col;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) col[r] = rb[i][r][j];
-        *(eas_h8*)(&Bs[(nc * 8 + j) * PITCH + kg * 8]) = col;
-      }
-    }
+  for (int i = 0; i < NB; ++i) {
+    const int r = (256 / BCH) * i + tid / BCH;
+    pb[i] = B + (size_t)r * ldb + bn;
+    lb[i] = r * BN + (((be >> 3) ^ bsw(r)) * 8) + (be & 7);
+  }
+  // how much of a unit of the last stage lies past the operand
+  constexpr int KL = (KT - 1) * BK;
+  auto lost_a = [&] { return eas_unit_lost<AT>(KL + ae, K); };
+  auto lost_b = [&](int i) {
+    const int k = KL + (256 / BCH) * i + tid / BCH;
+    return k >= K ? UB : k == K - 1 ? eas_unit_lost<BT>(bn, N) : 0;
   };
-  // edge tiles and the K tail: element loads with zero fill, written straight to LDS
-  // (rolled loops keep register pressure low; these tiles are few)
-  auto sstore_masked = [&](int buf, int k0) {
-    eas_op_t* As = As0 + buf * BM * PITCH;
-    eas_op_t* Bs = Bs0 + buf * BN * PITCH;
-#pragma unroll 1
-    for (int i = 0; i < A_IT; ++i) {
-      const int c = tid + NTHREADS * i, row = c / KC, kc = c % KC;
-      const int gm_ = m0 + row, gk = k0 + kc * 8;
-      eas_h8 v;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (gm_ < M && gk + e < K) ? (eas_op_t)A[(size_t)gm_ * K + gk + e] : (eas_op_t)0.0f;
-      *(eas_h8*)(&As[row * PITCH + kc * 8]) = v;
-    }
-#pragma unroll 1
-    for (int i = 0; i < B_IT; ++i) {
-      const int blk = tid + NTHREADS * i, kg = blk % KC, nc = blk / KC;
-      if (NBLK % NTHREADS != 0 && blk >= NBLK) break;
-      const int gn = n0 + nc * 8;
-#pragma unroll 1
-      for (int j = 0; j < 8; ++j) {
-        eas_h8 col;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int gk = k0 + kg * 8 + r;
-          col[r] = (gk < K && gn + j < N) ? (eas_op_t)B[(size_t)gk * ldb + gn + j] : (eas_op_t)0.0f;
-        }
-        *(eas_h8*)(&Bs[(nc * 8 + j) * PITCH + kg * 8]) = col;
-      }
-    }
-  };
-  eas_f32x16 acc[TI][TJ];
-#pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) acc[i][j] = (eas_f32x16){};
-
-  constexpr int KT = (K + BK - 1) / BK, KFULL = K / BK;
-  auto compute = [&](int kt) {
-    const eas_op_t* As = As0 + (kt & 1) * BM * PITCH;
-    const eas_op_t* Bs = Bs0 + (kt & 1) * BN * PITCH;
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      eas_h8 a[TI], b[TJ];
-      const int kk = ks * 16 + (lane >> 5) * 8;
-#pragma unroll
-      for (int i = 0; i < TI; ++i) a[i] = *(const eas_h8*)&As[(wm * 128 + i * 32 + (lane & 31)) * PITCH + kk];
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) b[j] = *(const eas_h8*)&Bs[(wn * 128 + j * 32 + (lane & 31)) * PITCH + kk];
-#pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = EAS_MFMA32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-  };
-  if (mn_full) {
-    // interior tile: full k-tiles stage through registers, loads issued before the current MFMAs
-    if (KFULL > 0) {
-      gload_fast(0);
-      sstore_regs(0);
+  eas_u32x4 xa[NA], xb[NB];  // the units of one stage
+  auto load_a = [&](int kt, int i) {
+    if (kt < KT - 1) {
+      xa[i] = eas_load_unit(pa[i] + (size_t)kt * BK);
     } else {
-      sstore_masked(0, 0);
+      const int lost = lost_a();
+      xa[i] = eas_load_unit(lost == UA ? A : pa[i] + (size_t)kt * BK - lost);
     }
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      const bool next_fast = kt + 1 < KFULL;
-      if (next_fast) gload_fast((kt + 1) * BK);
-      compute(kt);
-      if (next_fast) sstore_regs((kt + 1) & 1);
-      else if (kt + 1 < KT) sstore_masked((kt + 1) & 1, (kt + 1) * BK);  // the K tail
-      __syncthreads();
+  };
+  auto load_b = [&](int kt, int i) {
+    if (kt < KT - 1) {
+      xb[i] = eas_load_unit(pb[i] + (size_t)kt * BK * ldb);
+    } else {
+      const int lost = lost_b(i);
+      xb[i] = eas_load_unit(lost == UB ? B : pb[i] + (size_t)kt * BK * ldb - lost);
     }
-  } else {
-    sstore_masked(0, 0);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      compute(kt);
-      if (kt + 1 < KT) sstore_masked((kt + 1) & 1, (kt + 1) * BK);
-      __syncthreads();
+  };
+  auto finish = [&] {  // the last stage's units, before they are stored
+#pragma unroll
+    for (int i = 0; i < NA; ++i) xa[i] = eas_unit_end<AT>(xa[i], lost_a());
+#pragma unroll
+    for (int i = 0; i < NB; ++i) xb[i] = eas_unit_end<BT>(xb[i], lost_b(i));
+  };
+  auto put_a = [&](int s, int i) { eas_store_unit<AT>(As + s * STAGE_A + la[i], xa[i]); };
+  auto put_b = [&](int s, int i) { eas_store_unit<BT>(Bs + s * STAGE_B + lb[i], xb[i]); };
+  // fragments of k half ks: MI 16: A[row 16 i + l%16][k 32 ks + 8(l/16)..+7], B[k 32 ks + 8(l/16)..+7][col
+  // 16 j + l%16]; MI 32: A[row 32 i + l%32][k 16 ks + 8(l/32)..+7], B likewise
+  int fa_off[2][TI], fb_off[2][TJ];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const int r = wm * (BM / 2) + i * MI + (lane & (MI - 1));
+      const int c = MI == 16 ? 4 * ks + (lane >> 4) : 2 * ks + (lane >> 5);
+      fa_off[ks][i] = r * BK + ((c ^ asw(r)) * 8);
+    }
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      const int gq = lane >> 4, kq = lane & 15;
+      const int row = MI == 16 ? 32 * ks + 8 * gq + (kq >> 2) : 16 * ks + 8 * (gq >> 1) + (kq >> 2);
+      const int col = wn * (BN / 2) + j * MI + (MI == 16 ? 0 : 16 * (gq & 1)) + 4 * (kq & 3);
+      fb_off[ks][j] = row * BN + ((col >> 3) ^ bsw(row)) * 8 + (col & 7);
     }
   }
+  eas_h8 fa[2][TI], fb[2][TJ];
+  auto read_a = [&](int s, int ks, int i) { fa[ks][i] = *(const eas_h8*)(As + s * STAGE_A + fa_off[ks][i]); };
+  auto read_b = [&](int s, int ks, int j) {
+    const eas_op_t* bs = Bs + s * STAGE_B + fb_off[ks][j];
+    const eas_h4t lo = EAS_DS_TR16((EAS_LDS eas_h4t*)bs);
+    const eas_h4t hi = EAS_DS_TR16((EAS_LDS eas_h4t*)(bs + 4 * BN));
+    const eas_h4 l4 = __builtin_bit_cast(eas_h4, lo), h4 = __builtin_bit_cast(eas_h4, hi);
+    fb[ks][j] = (eas_h8){l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
+  };
+  eas_f32x16 acc32[MI == 32 ? TI : 1][MI == 32 ? TJ : 1];
+  eas_f32x4 acc16[MI == 16 ? TI : 1][MI == 16 ? TJ : 1];
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < TJ; ++j)
+    for (int j = 0; j < TJ; ++j) {
+      if constexpr (MI == 32) acc32[i][j] = (eas_f32x16){};
+      else acc16[i][j] = (eas_f32x4){};
+    }
+  auto mfma_row = [&](int ks, int i) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm * 128 + i * 32 + (r / 4) * 8 + (lane >> 5) * 4 + (r % 4);
-        const int col = n0 + wn * 128 + j * 32 + (lane & 31);
-        if (mn_full || (row < M && col < N)) C[(size_t)row * ldb + col] = (CT)acc[i][j][r];
+    for (int j = 0; j < TJ; ++j) {
+      if constexpr (MI == 32) acc32[i][j] = EAS_MFMA32(fa[ks][i], fb[ks][j], acc32[i][j], 0, 0, 0);
+      else acc16[i][j] = EAS_MFMA16(fa[ks][i], fb[ks][j], acc16[i][j], 0, 0, 0);
+    }
+  };
+  // stage kt, whose first fragments are in registers; xa, xb: stage kt+1's units, then kt+2's
+  auto stage = [&](int kt) {
+    const int s = kt & 1, sn = s ^ 1;
+    const bool next = kt + 1 < KT, more = kt + 2 < KT;
+    if (kt + 1 == KT - 1) finish();
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      read_a(s, 1, i);
+#pragma unroll
+      for (int j = i * TJ / TI; j < (i + 1) * TJ / TI; ++j) read_b(s, 1, j);
+      mfma_row(0, i);
+      if (next) {
+#pragma unroll
+        for (int u = i * NA / TI; u < (i + 1) * NA / TI; ++u) {
+          put_a(sn, u);
+          if (more) load_a(kt + 2, u);
+        }
+#pragma unroll
+        for (int u = i * NB / TI; u < (i + 1) * NB / TI; ++u) {
+          put_b(sn, u);
+          if (more) load_b(kt + 2, u);
+        }
       }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (next) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (next) {
+        read_a(sn, 0, i);
+#pragma unroll
+        for (int j = i * TJ / TI; j < (i + 1) * TJ / TI; ++j) read_b(sn, 0, j);
+      }
+      mfma_row(1, i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int i = 0; i < NB; ++i) load_b(0, i);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) load_a(0, i);
+  if (KT == 1) finish();
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    put_b(0, i);
+    if (KT > 1) load_b(1, i);
+  }
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    put_a(0, i);
+    if (KT > 1) load_a(1, i);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) read_b(0, 0, j);
+#pragma unroll
+  for (int i = 0; i < TI; ++i) read_a(0, 0, i);
+  for (int kt = 0; kt < KT; ++kt) stage(kt);
+  __builtin_amdgcn_s_waitcnt(EAS_WAITVM(0));  // as in eas_gemm_skinny_regs: no load is pending
+  const bool full = (m0 + BM <= M) && (n0 + BN <= N);
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      if constexpr (MI == 32) {
+        // lane l, register r of a 32x32 tile holds (row 8*(r/4) + 4*(l/32) + r%4, col l%32)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = m0 + wm * (BM / 2) + i * 32 + (r / 4) * 8 + (lane >> 5) * 4 + (r % 4);
+          const int col = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
+          if (full || (row < M && col < N)) C[(size_t)row * ldb + col] = (CT)acc32[i][j][r];
+        }
+      } else {
+        // lane l, register r of a 16x16 tile holds (row 4*(l/16) + r, col l%16)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = m0 + wm * (BM / 2) + i * 16 + (lane >> 4) * 4 + r;
+          const int col = n0 + wn * (BN / 2) + j * 16 + (lane & 15);
+          if (full || (row < M && col < N)) C[(size_t)row * ldb + col] = (CT)acc16[i][j][r];
+        }
+      }
+    }
 }
 
 // Origin of this workgroup's BM x BN tile: XCD-contiguous (workgroup w runs on XCD w % 8, so
@@ -1208,10 +1405,14 @@ extern "C" __global__ __launch_bounds__(256) void @NAME@(
   const bool dma_ok = OP_IN && (K % 2 == 0) && (ldb % 2 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) &&
                       ((uint64_t)M * K * 2 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 2 < (1ull << 31));
   const bool skinny_dma_ok = dma_ok && (K % 8 == 0) && (ldb % 8 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 16 == 0);
-  if (M <= SKINNY_M) {
+  // The grid says which tile the launch plan picked: the smallest whose count it is (where two tiles
+  // have the same count either covers C).  256 x 256 also for operands the DMA takes, on its 4-wave body.
+  auto count = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const int wgs = (int)gridDim.x;
+  if (M <= SKINNY_M && (M <= 64 || wgs != count(64, 64))) {
     // The launch plan gives one workgroup per 64 columns, or per 128 when that keeps the launch to
     // one round of CUs; the grid says which.  1, 2, 4 or 8 row tiles of 16.
-    const bool wide = (int)gridDim.x * 64 < N;
+    const bool wide = wgs * 64 < N;
     const int n0 = (int)blockIdx.x * (wide ? 128 : 64);
     if constexpr (OP_IN) {
       if (skinny_dma_ok) {
@@ -1233,27 +1434,42 @@ extern "C" __global__ __launch_bounds__(256) void @NAME@(
       }
     }
     // inputs the DMA cannot take (on a 128-column grid, 64 columns at a time)
-    if (M <= 16) {
-      eas_gemm_skinny_simple<AT, BT, CT, K, 1>(A, B, C, ldb, M, N, n0);
-      if (wide) eas_gemm_skinny_simple<AT, BT, CT, K, 1>(A, B, C, ldb, M, N, n0 + 64);
-    } else if (M <= 64) {
-      eas_gemm_skinny_simple<AT, BT, CT, K, 4>(A, B, C, ldb, M, N, n0);
-      if (wide) eas_gemm_skinny_simple<AT, BT, CT, K, 4>(A, B, C, ldb, M, N, n0 + 64);
-    } else {
-      eas_gemm_skinny_simple<AT, BT, CT, K, 8>(A, B, C, ldb, M, N, n0);
-      if (wide) eas_gemm_skinny_simple<AT, BT, CT, K, 8>(A, B, C, ldb, M, N, n0 + 64);
+    if (K < 8 || ldb < 8) {  // rows shorter than a 16-byte unit of 16-bit elements
+      eas_gemm_elementwise<AT, BT, CT, K, SKINNY_M, 128>(A, B, C, ldb, M, min(N, n0 + (wide ? 128 : 64)), 0, n0);
+      return;
+    }
+    for (int c0 = n0; c0 < min(N, n0 + (wide ? 128 : 64)); c0 += 64) {
+      if (M <= 16) eas_gemm_skinny_regs<AT, BT, CT, K, 1>(A, B, C, ldb, M, N, c0, smem);
+      else if (M <= 32) eas_gemm_skinny_regs<AT, BT, CT, K, 2>(A, B, C, ldb, M, N, c0, smem);
+      else if (M <= 64) eas_gemm_skinny_regs<AT, BT, CT, K, 4>(A, B, C, ldb, M, N, c0, smem);
+      else eas_gemm_skinny_regs<AT, BT, CT, K, 8>(A, B, C, ldb, M, N, c0, smem);
     }
     return;
   }
   int m0, n0;
-  eas_tile_origin(M, N, m0, n0);
   if constexpr (OP_IN) {
-    if (dma_ok) {
+    if (dma_ok && wgs == count(256, 256)) {
+      eas_tile_origin(M, N, m0, n0);
       eas_gemm_dma<CT, K>((const eas_op_t*)A, (const eas_op_t*)B, C, ldb, M, N, m0, n0, smem);
       return;
     }
   }
-  eas_gemm_regs<AT, BT, CT, K>(A, B, C, ldb, M, N, m0, n0, smem);
+  if (K < 8 || ldb < 8) {
+    for (int t = blockIdx.x; t < count(64, 64); t += wgs)
+      eas_gemm_elementwise<AT, BT, CT, K, 64, 64>(A, B, C, ldb, M, N, t % ((M + 63) / 64) * 64, t / ((M + 63) / 64) * 64);
+  } else if (wgs == count(64, 64)) {
+    eas_tile_origin<64, 64>(M, N, m0, n0);
+    eas_gemm_regs<AT, BT, CT, K, 64, 64>(A, B, C, ldb, M, N, m0, n0, smem);
+  } else if (wgs == count(128, 64)) {
+    eas_tile_origin<128, 64>(M, N, m0, n0);
+    eas_gemm_regs<AT, BT, CT, K, 128, 64>(A, B, C, ldb, M, N, m0, n0, smem);
+  } else if (wgs == count(128, 128)) {
+    eas_tile_origin<128, 128>(M, N, m0, n0);
+    eas_gemm_regs<AT, BT, CT, K, 128, 128>(A, B, C, ldb, M, N, m0, n0, smem);
+  } else {
+    eas_tile_origin(M, N, m0, n0);
+    eas_gemm_regs<AT, BT, CT, K, 256, 256>(A, B, C, ldb, M, N, m0, n0, smem);
+  }
 }
 """
 

@@ -1052,8 +1052,13 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
         groups = -(-n // p["skinny_n"])
         if m <= WIDE_M and groups > compute_units:
             groups = -(-n // (2 * p["skinny_n"]))
+        # Operands the DMA entries cannot take run 64 x 64 register tiles above 64 rows (128 x 4096 x
+        # 1024 f32 on 64 skinny groups 17.5 us, on 128 tiles 7.8; 100 x 4097 x 1023 f16 15.0 and 8.9).
         other = None
-        if m > SKINNY_CUT and p.get("pp_entry") and _dma_fits(p, runtime_args, K, ldb, m, n_lo, n):
+        fits = p.get("pp_entry") and _dma_fits(p, runtime_args, K, ldb, m, n_lo, n)
+        if m > 64 and not fits:
+            other = LaunchPlan((tiles64, 1, 1), (p["threads"], 1, 1), hidden)
+        elif m > SKINNY_CUT and fits:
             if choice == "tile128" or (choice == "auto" and groups > compute_units):
                 other = LaunchPlan((tiles128, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t128_entry"])
             elif choice == "tile128x256":
@@ -1089,7 +1094,27 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
         if choice == "tile128" or small:
             return LaunchPlan((tiles128, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t128_entry"])
         return LaunchPlan((tiles, 1, 1), (p["pp_threads"], 1, 1), hidden, entry=p["pp_entry"])
+    if choice != "4wave" or not (p.get("pp_entry") and _dma_fits(p, runtime_args, K, ldb, m, n_lo, n)):
+        tiles = _register_tiles(m, n, compute_units)
     return LaunchPlan((tiles, 1, 1), (p["threads"], 1, 1), hidden)
+
+
+# Tiles of the main entry's register body (operands the DMA cannot take) and the relative time of one
+# round of them, one workgroup per CU.  Measured per 64 k, f16 with odd rows (f32 operands in
+# brackets): 64 x 64 0.50 us (0.58), 128 x 64 0.62 (0.78), 128 x 128 0.89 (1.03), 256 x 256 1.7 (2.0-2.4).
+REGISTER_TILES = ((64, 64, 10), (128, 64, 13), (128, 128, 18), (256, 256, 36))
+
+
+def _register_tiles(m: int, n: int, cus: int) -> int:
+    """Workgroups of the register tile with the least rounds x time per round (the larger tile of
+    equals, which reads less); the kernel tells the tile from the count."""
+    best = None
+    for bm, bn, w in REGISTER_TILES:
+        t = -(-m // bm) * -(-n // bn)
+        cost = -(-t // cus) * w
+        if best is None or cost <= best[0]:
+            best = (cost, t)
+    return best[1]
 
 
 _ENTRY_CHOICES = ("auto", "8wave", "tile128", "tile128x256", "tile128x64", "tile64", "4wave")

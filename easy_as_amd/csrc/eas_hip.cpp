@@ -682,6 +682,22 @@ bool dma_fits(uint64_t a_ptr, uint64_t b_ptr, uint64_t K, uint64_t ldb, uint64_t
 
 uint64_t cdiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
+// Workgroups of the main entry's register body (operands the DMA cannot take): the tile with the
+// least rounds x time per round, the larger of equals.  The kernel tells the tile from the count.
+uint64_t register_tiles(uint64_t m, uint64_t n, uint64_t cus) {
+  static const struct {
+    uint64_t bm, bn, w;  // w: relative time of one round (gemm_lift.REGISTER_TILES holds the measurements)
+  } kTiles[] = {{64, 64, 10}, {128, 64, 13}, {128, 128, 18}, {256, 256, 36}};
+  u128 best = 0;
+  uint64_t wgs = 0;
+  for (const auto& t : kTiles) {
+    const uint64_t n_tiles = cdiv(m, t.bm) * cdiv(n, t.bn);
+    const u128 cost = (u128)cdiv(n_tiles, cus) * t.w;
+    if (!wgs || cost <= best) best = cost, wgs = n_tiles;
+  }
+  return wgs;
+}
+
 }  // namespace
 
 int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g, const void* kernarg,
@@ -773,7 +789,11 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g
     uint64_t grp = cdiv(n, g->skinny_n);
     if (m <= g->wide_m && grp > cus) grp = cdiv(n, 2ull * g->skinny_n);
     pick(EAS_HIP_GEMM_MAIN, grp, g->threads);
-    if (m > g->skinny_cut && has(EAS_HIP_GEMM_PP) && fits()) {
+    // Operands the DMA entries cannot take run 64 x 64 register tiles above 64 rows.
+    const bool dma = has(EAS_HIP_GEMM_PP) && fits();
+    if (m > 64 && !dma) {
+      wgs = tiles64;
+    } else if (m > g->skinny_cut && dma) {
       if (ch == kTile128 || (ch == kAuto && grp > cus)) pick(EAS_HIP_GEMM_T128, tiles128, g->t128_threads);
       else if (ch == kTile128x256) pick(EAS_HIP_GEMM_T128X256, tiles128x256, g->t128_threads);
       else if (ch == kTile128x64) pick(EAS_HIP_GEMM_T128X64, tiles128x64, g->t128_threads);
@@ -795,6 +815,8 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g
     else if (ch == kTile128x64 || tiny) pick(EAS_HIP_GEMM_T128X64, tiles128x64, g->t128_threads);
     else if (ch == kTile128 || small) pick(EAS_HIP_GEMM_T128, tiles128, g->t128_threads);
     else pick(EAS_HIP_GEMM_PP, tiles, g->pp_threads);
+  } else if (ch != k4Wave || !has(EAS_HIP_GEMM_PP) || !fits()) {
+    wgs = register_tiles(m, n, cus);
   }
   if (!has(entry))
     return fail(EAS_HIP_ERR_INVALID, "GEMM entry %s%s is not in the code object", g->entry, kGemmSuffix[entry]);
