@@ -904,11 +904,12 @@ PyObject* py_launch_timed(PyObject*, PyObject* args, PyObject* kwargs) {
 // ---- the call memo's launch, in one native call ---------------------------------------
 //
 // A repeated eas call with the same argument types (torch GPU tensors and Python scalars, no
-// launch options) launches what its first call planned, but on the arguments it is given now.
+// launch options but a grid) launches what its first call planned, but on the arguments it is given now.
 // fast_make records, per argument, what the first call's specialisation expects; fast_call
 // checks the new arguments against it (exact types, the tensor's dtype object, is_cuda,
 // contiguity), packs the device pointers and scalars, plans the dispatch from N as launch_tg
-// would (cached for the last N), launches on torch's current stream of the last torch tensor's
+// would (cached for the last N) or from the call's grid (a lifted GEMM also from its arguments and
+// the buffers' lengths, on every call), launches on torch's current stream of the last torch tensor's
 // device (the default stream when every buffer is an eas.Tensor) and, when asynchronous, returns a
 // pending capsule of the stream's batch.  Any argument it does
 // not take returns NotImplemented before anything is launched, and the caller takes its full
@@ -927,7 +928,7 @@ struct Fast {
   eas_hip_kernel* k = nullptr;
   eas_hip_launch_shape shape{};
   std::vector<FastArg> args;
-  int n_index = -1;                 // position of the u32 argument N
+  int n_index = -1;                 // position of the u32 argument N (-1: every call gives its grid)
   bool by_groups = true;            // SPMD: N lanes are ceil(N / BLOCK) programs; thread mode: N threads
   bool sync = true;
   int batch = kBatchLaunches;
@@ -962,7 +963,8 @@ void fast_destructor(PyObject* cap) {
 // fast_make(kernel, specs, n_index, sync, batch, tensor_type, raw_stream, eas_type) -> fast capsule.
 // specs: one (kind, expect) per kernel argument, kind 0 torch tensor (expect: its torch dtype),
 // 1 u32 (int), 2 f32 (float), 3 bool, 4 eas.Tensor on the GPU (expect: its NumPy dtype); the kernel
-// must have an SPMD or thread-mode launch shape.
+// must have a launch shape, an SPMD or thread-mode one for launches sized by N.  n_index -1: the
+// launches are sized by the grid each call gives.
 PyObject* py_fast_make(PyObject*, PyObject* args) {
   PyObject *kcap, *specs, *tensor_type, *raw_stream, *eas_type;
   int n_index, sync, batch;
@@ -974,7 +976,7 @@ PyObject* py_fast_make(PyObject*, PyObject* args) {
   eas_hip_launch_shape s;
   int rc = eas_hip_kernel_get_shape(k, &s);
   if (rc) return raise_status(rc);
-  if (s.kind != EAS_HIP_KIND_SPMD && s.kind != EAS_HIP_KIND_THREAD) {
+  if (s.kind != EAS_HIP_KIND_SPMD && s.kind != EAS_HIP_KIND_THREAD && (s.kind != EAS_HIP_KIND_GEMM || n_index >= 0)) {
     PyErr_SetString(PyExc_ValueError, "fast_make: the kernel needs an SPMD or thread-mode launch shape");
     return nullptr;
   }
@@ -1008,7 +1010,7 @@ PyObject* py_fast_make(PyObject*, PyObject* args) {
     off += size;
   }
   Py_DECREF(seq);
-  if (ok && (n_index < 0 || n_index >= (int)f->args.size() || f->args[n_index].kind != kFastU32)) {
+  if (ok && n_index != -1 && (n_index < 0 || n_index >= (int)f->args.size() || f->args[n_index].kind != kFastU32)) {
     PyErr_SetString(PyExc_ValueError, "fast_make: N must be a u32 argument");
     ok = false;
   }
@@ -1043,6 +1045,7 @@ PyObject* g_s_is_cuda = nullptr;
 PyObject* g_s_is_contiguous = nullptr;
 PyObject* g_s_data_ptr = nullptr;
 PyObject* g_s_get_device = nullptr;
+PyObject* g_s_nbytes = nullptr;
 PyObject* g_s_device_attr = nullptr;  // eas.Tensor._device
 PyObject* g_s_dtype_attr = nullptr;   // eas.Tensor._dtype
 PyObject* g_s_hip_attr = nullptr;     // eas.Tensor._hip (its storage; .buf the buffer capsule)
@@ -1057,12 +1060,12 @@ int call_true(PyObject* obj, PyObject* name) {
   return t;
 }
 
-// fast_call(fast, args: tuple) -> None (launched and, if synchronous, done), a pending capsule
-// (asynchronous), or NotImplemented (an argument this specialisation's fast path does not take;
-// nothing was launched).
+// fast_call(fast, args: tuple, grid: tuple = None) -> None (launched and, if synchronous, done), a
+// pending capsule (asynchronous), or NotImplemented (an argument or grid this specialisation's fast
+// path does not take; nothing was launched).  grid: 1..3 ints, the launch's programs or threadgroups.
 PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
-  if (nargv != 2 || !PyTuple_Check(argv[1])) {
-    PyErr_SetString(PyExc_TypeError, "fast_call(fast, args: tuple)");
+  if (nargv < 2 || nargv > 3 || !PyTuple_Check(argv[1])) {
+    PyErr_SetString(PyExc_TypeError, "fast_call(fast, args: tuple, grid: tuple = None)");
     return nullptr;
   }
   auto* f = static_cast<Fast*>(PyCapsule_GetPointer(argv[0], kFastCap));
@@ -1070,6 +1073,28 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
   PyObject* args = argv[1];
   const size_t n = f->args.size();
   if ((size_t)PyTuple_GET_SIZE(args) != n) Py_RETURN_NOTIMPLEMENTED;
+  uint64_t groups[3] = {1, 1, 1};
+  const bool by_grid = nargv == 3;
+  if (by_grid != (f->n_index < 0)) Py_RETURN_NOTIMPLEMENTED;
+  if (by_grid) {
+    PyObject* grid = argv[2];
+    if (!PyTuple_CheckExact(grid)) Py_RETURN_NOTIMPLEMENTED;
+    const Py_ssize_t dims = PyTuple_GET_SIZE(grid);
+    if (dims < 1 || dims > 3) Py_RETURN_NOTIMPLEMENTED;
+    for (Py_ssize_t i = 0; i < dims; ++i) {
+      PyObject* d = PyTuple_GET_ITEM(grid, i);
+      if (!PyLong_CheckExact(d)) Py_RETURN_NOTIMPLEMENTED;
+      groups[i] = PyLong_AsUnsignedLongLong(d);
+      if (PyErr_Occurred()) {
+        PyErr_Clear();  // negative or huge: the full path reports it
+        Py_RETURN_NOTIMPLEMENTED;
+      }
+      if (groups[i] == 0) Py_RETURN_NOTIMPLEMENTED;  // nothing to run: the full path checks the arguments
+    }
+  }
+  const bool gemm = f->shape.kind == EAS_HIP_KIND_GEMM;
+  uint64_t lengths[64];  // a lifted GEMM's buffer lengths in bytes, by argument
+  if (gemm && n > 64) Py_RETURN_NOTIMPLEMENTED;
   uint8_t blob[512];
   const size_t arg_bytes = f->shape.arg_bytes, total = (arg_bytes + 3) / 4 * 4 + 4 * (size_t)f->shape.hidden;
   if (total > sizeof(blob)) Py_RETURN_NOTIMPLEMENTED;
@@ -1099,6 +1124,13 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
       if (PyErr_Occurred()) return nullptr;
       memcpy(blob + a.offset, &ptr, 8);
       last_tensor = obj;
+      if (gemm) {
+        PyObject* nb = PyObject_GetAttr(obj, g_s_nbytes);
+        if (!nb) return nullptr;
+        lengths[i] = PyLong_AsUnsignedLongLong(nb);
+        Py_DECREF(nb);
+        if (PyErr_Occurred()) return nullptr;
+      }
       continue;
     }
     if (a.kind == kFastEasTensor) {
@@ -1128,6 +1160,7 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
       continue;
     }
     if ((PyObject*)Py_TYPE(obj) != a.expect) Py_RETURN_NOTIMPLEMENTED;
+    lengths[i & 63] = 0;
     if (a.kind == kFastU32) {
       unsigned long long v = PyLong_AsUnsignedLongLong(obj);
       if (PyErr_Occurred() || v > 0xFFFFFFFFull) {
@@ -1146,8 +1179,12 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
       blob[a.offset] = obj == Py_True ? 1 : 0;
     }
   }
-  if (nval == 0) Py_RETURN_NONE;  // a zero extent launches nothing
-  if (!f->have_plan || f->plan_n != nval) {
+  if (!by_grid && nval == 0) Py_RETURN_NONE;  // a zero extent launches nothing
+  if (by_grid && !gemm) {
+    static const uint32_t kAuto[3] = {0, 0, 0};
+    int rc = eas_hip_plan_dispatch(&f->shape, 1, groups, kAuto, f->grid, f->block, f->hidden, EAS_HIP_MAX_HIDDEN);
+    if (rc) Py_RETURN_NOTIMPLEMENTED;  // the full path reports the size error
+  } else if (!by_grid && (!f->have_plan || f->plan_n != nval)) {
     const uint32_t block = f->shape.block_size;
     const uint64_t size[3] = {f->by_groups ? (nval + block - 1) / block : nval, 1, 1};
     static const uint32_t kAuto[3] = {0, 0, 0};
@@ -1172,7 +1209,13 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
     Py_DECREF(sobj);
     if (PyErr_Occurred()) return nullptr;
   }
-  int rc = eas_hip_launch(f->k, blob, total, f->grid, f->block, 0, stream, 1);
+  int rc;
+  if (gemm) {
+    rc = eas_hip_launch_threadgroups(f->k, blob, arg_bytes, lengths, (int)n, groups, nullptr, stream, 1);
+    if (rc == EAS_HIP_ERR_INVALID) Py_RETURN_NOTIMPLEMENTED;  // refused before a launch: the full path reports it
+  } else {
+    rc = eas_hip_launch(f->k, blob, total, f->grid, f->block, 0, stream, 1);
+  }
   if (rc) return raise_status(rc);
   if (f->sync) {
     Py_BEGIN_ALLOW_THREADS
@@ -1528,7 +1571,7 @@ PyMethodDef kMethods[] = {
     {"synchronize", py_synchronize, METH_VARARGS, "Wait for a pending launch and drop its keepalives."},
     {"fast_make", py_fast_make, METH_VARARGS, "The call memo's native launch for one specialisation."},
     {"fast_call", (PyCFunction)(void (*)(void))py_fast_call, METH_FASTCALL,
-     "fast_call(fast, args): launch the memoized specialisation, or NotImplemented."},
+     "fast_call(fast, args, grid=None): launch the memoized specialisation, or NotImplemented."},
     {"pending_info", py_pending_info, METH_VARARGS, "Completion batch of a pending launch (stream, launches, closed)."},
     {"queue_synchronize", py_queue_synchronize, METH_VARARGS, "Wait for a stream (default: whole device)."},
     {"dlpack_import", py_dlpack_import, METH_VARARGS, "Zero-copy import of a kDLROCM DLPack capsule."},
@@ -1546,6 +1589,7 @@ PyMODINIT_FUNC PyInit__hip(void) {
   g_s_is_contiguous = PyUnicode_InternFromString("is_contiguous");
   g_s_data_ptr = PyUnicode_InternFromString("data_ptr");
   g_s_get_device = PyUnicode_InternFromString("get_device");
+  g_s_nbytes = PyUnicode_InternFromString("nbytes");
   g_s_device_attr = PyUnicode_InternFromString("_device");
   g_s_dtype_attr = PyUnicode_InternFromString("_dtype");
   g_s_hip_attr = PyUnicode_InternFromString("_hip");

@@ -91,6 +91,10 @@ class Kernel:
         self._memo: dict[Any, tuple[CompiledKernel, dict[str, Any], bool]] = {}
         # the runtime's one-native-call launch of a memoized specialisation, by keyword items
         self._fast: dict[Any, Callable[[tuple[Any, ...]], Any]] = {}
+        # the same for calls that give their grid as a tuple: keyed by the other keyword items, the
+        # grid is an argument of the launch
+        self._grid_fast: dict[Any, Callable[[tuple[Any, ...], tuple[int, ...]], Any]] = {}
+        self._grid_kw = self._memo_kw | {"_grid", "_tptg"}
 
     def _set_autotune_spec(self, spec: AutotuneSpec) -> None:
         self._autotune_spec = spec
@@ -258,7 +262,10 @@ class Kernel:
 
     def __call__(self, /, *args: Any, **kwargs: Any) -> None:
         key = None
-        if self._memo_ok and len(args) == self._n_lead and self._autotune_spec is None:
+        if "_grid" in kwargs:
+            if self._call_grid(args, kwargs):
+                return
+        elif self._memo_ok and len(args) == self._n_lead and self._autotune_spec is None:
             try:
                 kw = tuple(kwargs.items())
                 fast = self._fast.get(kw)
@@ -290,6 +297,34 @@ class Kernel:
                     if len(self._fast) >= _MEMO_LIMIT:
                         self._fast.clear()
                     self._fast[key[0]] = fast
+
+    def _call_grid(self, args: tuple[Any, ...], kwargs: dict[str, Any]) -> bool:
+        """A call with ``_grid`` given as a tuple, on the runtime's one-native-call launch if an
+        earlier call of its shape made one; else the full path, which makes one for the calls after
+        it.  False: not such a call, nothing done."""
+        grid = kwargs["_grid"]
+        if type(grid) is not tuple or not self._memo_ok or len(args) != self._n_lead \
+                or self._autotune_spec is not None or not kwargs.keys() <= self._grid_kw \
+                or type(kwargs.get("_tptg", ())) is not tuple:
+            return False
+        kw = tuple([item for item in kwargs.items() if item[0] != "_grid"])
+        try:
+            fast = self._grid_fast.get(kw)
+        except TypeError:  # a keyword value that is not hashable
+            return False
+        if fast is not None and fast(args, grid) is not NotImplemented:
+            return True
+        ck, meta, runtime_args, opts, _ = self._prepare(args, dict(kwargs))
+        rt = get_runtime()
+        rt.run(ck, runtime_args, meta, **opts)
+        make = getattr(rt, "grid_launcher", None)
+        if fast is None and callable(make):
+            fast = make(ck, self._names[:self._n_lead], args, opts["sync"])
+            if fast is not None:
+                if len(self._grid_fast) >= _MEMO_LIMIT:
+                    self._grid_fast.clear()
+                self._grid_fast[kw] = fast
+        return True
 
     def to_hip(self, /, *args: Any, **kwargs: Any) -> str:
         """The generated gfx950 HIP C++ source for this specialisation (reference: ``to_msl``)."""

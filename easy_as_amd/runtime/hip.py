@@ -361,18 +361,39 @@ class HipRuntime:
         EAS_MAX_IN_FLIGHT bound) and returns None, or returns NotImplemented without launching
         when an argument does not match (another type, dtype or device kind, a non-contiguous
         tensor, a scalar out of range): the caller then takes the full path."""
-        from ..tensor import Tensor as EasTensor
-
-        torch = self._torch_mod()
         geo = ck.geometry
         if geo is None or geo.kind not in ("spmd", "thread") or grid_ndim(ck.ir) > 1:
             return None
+        specs = self._fast_specs(ck, names, args)
+        n_index = next((i for i, a in enumerate(ck.ir.args) if a.name == "N"), None)
+        if specs is None or n_index is None or specs[n_index][0] != 1:
+            return None
+        return self._fast_launch(ck, specs, n_index, sync)
+
+    def grid_launcher(self, ck: Any, names: tuple[str, ...], args: tuple[Any, ...], sync: bool) -> Any:
+        """``fast_launcher`` for launches whose ``_grid`` is a tuple of ints: the returned callable
+        takes the call's arguments and its grid.  Every kernel kind, a lifted GEMM (whose plan the
+        native layer makes from its arguments on each call) with torch tensors only."""
+        geo = ck.geometry
+        if geo is None or geo.kind not in ("spmd", "thread", "gemm"):
+            return None
+        specs = self._fast_specs(ck, names, args)
+        if specs is None or (geo.kind == "gemm" and any(kind == 4 for kind, _ in specs)):
+            return None
+        return self._fast_launch(ck, specs, -1, sync)
+
+    def _fast_specs(self, ck: Any, names: tuple[str, ...], args: tuple[Any, ...]) -> list[tuple[int, Any]] | None:
+        """Per-argument (kind, expected dtype or type) of a native fast launch, None when an
+        argument is of a kind it does not take."""
+        from ..tensor import Tensor as EasTensor
+
+        torch = self._torch_mod()
         mod = self._mod()
         if not callable(getattr(mod, "fast_make", None)) or tuple(a.name for a in ck.ir.args) != tuple(names):
             return None
         scalar_kinds = {DType.U32: (1, int), DType.F32: (2, float), DType.BOOL: (3, bool)}
-        specs, n_index = [], None
-        for i, (a, v) in enumerate(zip(ck.ir.args, args)):
+        specs: list[tuple[int, Any]] = []
+        for a, v in zip(ck.ir.args, args):
             if a.kind == "buffer":
                 if type(v) is EasTensor:
                     want = _NP_DTYPES.get(a.dtype)
@@ -389,10 +410,12 @@ class HipRuntime:
             if kind is None or type(v) is not kind[1]:
                 return None
             specs.append(kind)
-            if a.name == "N" and kind[0] == 1:
-                n_index = i
-        if n_index is None:
-            return None
+        return specs
+
+    def _fast_launch(self, ck: Any, specs: list[tuple[int, Any]], n_index: int, sync: bool) -> Any:
+        from ..tensor import Tensor as EasTensor
+
+        torch, mod = self._torch_mod(), self._mod()
         limit = self._max_pending()
         # without torch every buffer is an eas.Tensor, and the launch goes on the default stream
         tensor_type, streams = (torch.Tensor, self._stream_getter()) if torch is not None else (type(None), id)
@@ -400,8 +423,8 @@ class HipRuntime:
                              tensor_type, streams, EasTensor)
         call, pending, synchronize = mod.fast_call, self._pending, mod.synchronize
 
-        def launch(call_args: tuple[Any, ...]) -> Any:
-            p = call(fast, call_args)
+        def launch(*call_args: Any) -> Any:  # the arguments' tuple, and the grid of a launch sized by one
+            p = call(fast, *call_args)
             if p is None or p is NotImplemented:
                 return p
             pending.append(p)
