@@ -87,6 +87,10 @@ static __device__ __forceinline__ eas_rsrc eas_make_rsrc(const void* base, uint3
   r[3] = 0x00020000;
   return r;
 }
+template <bool V>
+struct eas_bool_c {  // a compile-time flag passed as a value (to select a loop version)
+  static constexpr bool value = V;
+};
 // 16 bytes per lane, HBM -> LDS; lane i writes LDS bytes [lds + 16 i, lds + 16 i + 16).
 // Issued as asm so the compiler does not add vmcnt(0) before every LDS read; the
 // pipelines count their own loads with EAS_WAITVM.
@@ -363,10 +367,6 @@ static __device__ __forceinline__ void eas_gemm_dma(const eas_op_t* __restrict__
 // MI selects the MFMA: 32 (v_mfma_f32_32x32x16: each wave's 128 x 64 as 4 x 2 tiles of 32 x 32,
 // two k-steps of 16 per stage) or 16 (v_mfma_f32_16x16x32: 8 x 4 tiles of 16 x 16, one k-step of
 // 32 per stage; fewer accumulator bytes move through the MFMA per flop).  Same LDS reads per stage.
-template <bool V>
-struct eas_bool_c {  // a compile-time flag passed as a value (to select a loop version)
-  static constexpr bool value = V;
-};
 template <typename CT, int K, int MI = 32>
 static __device__ __forceinline__ void eas_gemm_pp(const eas_op_t* __restrict__ A, const eas_op_t* __restrict__ B,
                                                    CT* __restrict__ C, int ldb, int M, int N, int m0, int n0,
@@ -1623,10 +1623,11 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@(
   const int gsize = GROUP_M * tilesN, g = t / gsize, first_m = g * GROUP_M;
   const int gm = min(tilesM - first_m, GROUP_M);
   const int m0 = (first_m + (t % gsize) % gm) * BM, n0 = ((t % gsize) / gm) * BN;
-  const bool dma_ok = (K % 4 == 0) && (ldb % 4 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 16 == 0) &&
-                      ((uint64_t)M * K * 4 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 4 < (1ull << 31));
+  // rows of any length from 4 columns on: the DMA takes 16 bytes from any 4-byte aligned address
+  const bool dma_ok = ldb >= 4 && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) && ((uint64_t)M * K * 4 < (1ull << 31)) &&
+                      (((uint64_t)(K - 1) * ldb + N) * 4 < (1ull << 31));
   if (!dma_ok) {
-    // rows not 16-byte aligned: each of 256 threads accumulates a 4 x 4 block with plain fmas
+    // operands past the DMA's 2 GiB range, or under 4 columns: each of 256 threads accumulates a 4 x 4 block with plain fmas
     if (tid >= 256) return;
     const int r0 = m0 + (tid >> 4) * 4, c0 = n0 + (tid & 15) * 4;
     float acc[4][4] = {};
@@ -1652,10 +1653,15 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@(
     // producer: the DMA (1 KB per instruction, 2 A + 2 B per wave per stage, q = 2 pw + i)
     //   A stage [64 rows][32 k]: rows 8q + lane/8, 16-byte chunk lane%8 stored at chunk ^ ((row/2)%8)
     //   B stage [32 k][64 n]:    rows 4q + lane/16, chunk lane%16 stored at chunk ^ 8((row/16)%2)
-    // Rows past M and columns past N load zeros (they are never stored), so every address a load
-    // reads, lane offset plus stage offset, lies inside A or B.  The last stage of a K that is not
-    // a multiple of BK loads zeros past K; stages past K load zeros into a slot nobody reads, so
-    // every stage issues 4 loads and the count at each barrier is the same.
+    // Rows past M and chunks past N load zeros (they are never stored), and a chunk that straddles N
+    // reads on into B's next row, so in every stage but the last each address a load reads, lane
+    // offset plus stage offset, lies inside A or B.  The last stage keeps the whole offset in the
+    // lane, where the range check (per dword) sees all of it: it loads zeros past K and past the
+    // end of B, but for the A chunk that straddles K: the consumers mask what it holds past K.
+    // Stages past K load zeros into a slot nobody reads, so every stage issues the same loads and
+    // the count at each barrier is the same.  The loop has no VALU: with two adds a stage for edge
+    // tiles, 2048 x 2047 x 2048 ran 127.2 us against 120.0, and with selects between the forms
+    // 2048^3 127.6 against 119.7.
     const int pw = wave - 4;
     const eas_rsrc ra = eas_make_rsrc(A, (uint32_t)M * (uint32_t)K * 4u);
     const eas_rsrc rb = eas_make_rsrc(B, ((uint32_t)(K - 1) * (uint32_t)ldb + (uint32_t)N) * 4u);
@@ -1666,11 +1672,13 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@(
     for (int i = 0; i < 2; ++i) {
       const int q = pw * 2 + i;
       const int r = 8 * q + (lane >> 3), lc = (lane & 7) ^ ((r >> 1) & 7);
-      a_off[i] = m0 + r < M ? ((uint32_t)(m0 + r) * (uint32_t)K + (uint32_t)(lc * 4)) * 4u : 0x80000000u;
-      a_tail[i] = lc * 4 >= KLAST ? 0x80000000u : a_off[i];
+      const uint32_t a_raw = ((uint32_t)(m0 + r) * (uint32_t)K + (uint32_t)(lc * 4)) * 4u;
+      a_off[i] = m0 + r < M ? a_raw : 0x80000000u;
+      a_tail[i] = (m0 + r < M && lc * 4 < KLAST) ? a_raw + (uint32_t)((KT - 1) * BK * 4) : 0x80000000u;
       const int rr = 4 * q + (lane >> 4), lcb = (lane & 15) ^ (8 * ((rr >> 4) & 1));
-      b_off[i] = n0 + lcb * 4 < N ? (uint32_t)(n0 + lcb * 4) * 4u + (uint32_t)rr * (uint32_t)ldb * 4u : 0x80000000u;
-      b_tail[i] = rr >= KLAST ? 0x80000000u : b_off[i];
+      const uint32_t b_raw = (uint32_t)(n0 + lcb * 4) * 4u + (uint32_t)rr * (uint32_t)ldb * 4u;
+      b_off[i] = n0 + lcb * 4 < N ? b_raw : 0x80000000u;
+      b_tail[i] = rr < KLAST ? b_raw + (uint32_t)((KT - 1) * BK * 4) * (uint32_t)ldb : 0x80000000u;
     }
     auto dma = [&](int kt) {
       const uint32_t st = lds0 + (uint32_t)((kt % NSTAGE) * STF) * 4u;
@@ -1681,11 +1689,11 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@(
           eas_dma16s(ra, 0x80000000u, 0u, st + (pw * 2 + i) * 1024);
           eas_dma16s(rb, 0x80000000u, 0u, st + AST * 4 + (pw * 2 + i) * 1024);
         }
-      } else if (K % BK != 0 && kt == KT - 1) {
+      } else if (kt == KT - 1) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          eas_dma16s(ra, a_tail[i], sa, st + (pw * 2 + i) * 1024);
-          eas_dma16s(rb, b_tail[i], sb, st + AST * 4 + (pw * 2 + i) * 1024);
+          eas_dma16s(ra, a_tail[i], 0u, st + (pw * 2 + i) * 1024);
+          eas_dma16s(rb, b_tail[i], 0u, st + AST * 4 + (pw * 2 + i) * 1024);
         }
       } else {
 #pragma unroll
@@ -1755,6 +1763,15 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@(
     __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
+  // the last stage of a K that is not a multiple of 4: what the straddling chunk holds past K
+  auto mask_tail = [&](eas_f32x4 (&a)[4]) {
+    if constexpr (K % 4 != 0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[u][e] = (KT - 1) * BK + 4 * u + e + 16 * c >= K ? 0.0f : a[u][e];
+    }
+  };
   __syncthreads();  // stage 0 landed
   eas_f32x4 a0[4], a1[4];
   float b0[16], b1[16];
@@ -1764,8 +1781,10 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@(
     step(kt, a0, b0, a1, b1);
     step(kt + 1, a1, b1, a0, b0);
   }
+  if constexpr (KT % 2 != 0) mask_tail(a0);
   if constexpr (KT % 2 == 0) {
     step(KT - 2, a0, b0, a1, b1);
+    mask_tail(a1);
     mfmas(a1, b1);
   } else {
     mfmas(a0, b0);
@@ -1806,8 +1825,9 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
   const int gsize = GROUP_M * tilesN, g = t / gsize, first_m = g * GROUP_M;
   const int gm = min(tilesM - first_m, GROUP_M);
   const int m0 = (first_m + (t % gsize) % gm) * BM, n0 = ((t % gsize) / gm) * BN;
-  const bool dma_ok = (K % 4 == 0) && (ldb % 4 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 16 == 0) &&
-                      ((uint64_t)M * K * 4 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 4 < (1ull << 31));
+  // rows of any length from 4 columns on: the DMA takes 16 bytes from any 4-byte aligned address
+  const bool dma_ok = ldb >= 4 && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) && ((uint64_t)M * K * 4 < (1ull << 31)) &&
+                      (((uint64_t)(K - 1) * ldb + N) * 4 < (1ull << 31));
   if (!dma_ok) {
     // guard for operands the launch plan could not see: one f32 dot product per element
     for (int e = tid; e < BM * BN; e += 512) {
@@ -1823,10 +1843,7 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
     // producer: the DMA (1 KB per instruction, 4 A + 4 B per wave per stage, q = 4 pw + i)
     //   A stage [128 rows][32 k]: rows 8q + lane/8, chunk lane%8 stored at chunk ^ ((row/2)%8)
     //   B stage [32 k][128 n]:    rows 2q + lane/32, chunk lane%32 stored at chunk ^ 8((row/16)%2)
-    // Rows past M and columns past N load zeros (they are never stored), so every address a load
-    // reads, lane offset plus stage offset, lies inside A or B.  The last stage of a K that is not
-    // a multiple of BK loads zeros past K; stages past K load zeros into a slot nobody reads, so
-    // every stage issues 8 loads and the count at each barrier is the same.
+    // Range and ends of rows as in the 64 x 64 entry.
     const int pw = wave - 4;
     const eas_rsrc ra = eas_make_rsrc(A, (uint32_t)M * (uint32_t)K * 4u);
     const eas_rsrc rb = eas_make_rsrc(B, ((uint32_t)(K - 1) * (uint32_t)ldb + (uint32_t)N) * 4u);
@@ -1837,11 +1854,13 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
     for (int i = 0; i < 4; ++i) {
       const int q = pw * 4 + i;
       const int r = 8 * q + (lane >> 3), lc = (lane & 7) ^ ((r >> 1) & 7);
-      a_off[i] = m0 + r < M ? ((uint32_t)(m0 + r) * (uint32_t)K + (uint32_t)(lc * 4)) * 4u : 0x80000000u;
-      a_tail[i] = lc * 4 >= KLAST ? 0x80000000u : a_off[i];
+      const uint32_t a_raw = ((uint32_t)(m0 + r) * (uint32_t)K + (uint32_t)(lc * 4)) * 4u;
+      a_off[i] = m0 + r < M ? a_raw : 0x80000000u;
+      a_tail[i] = (m0 + r < M && lc * 4 < KLAST) ? a_raw + (uint32_t)((KT - 1) * BK * 4) : 0x80000000u;
       const int rr = 2 * q + (lane >> 5), lcb = (lane & 31) ^ (8 * ((rr >> 4) & 1));
-      b_off[i] = n0 + lcb * 4 < N ? (uint32_t)(n0 + lcb * 4) * 4u + (uint32_t)rr * (uint32_t)ldb * 4u : 0x80000000u;
-      b_tail[i] = rr >= KLAST ? 0x80000000u : b_off[i];
+      const uint32_t b_raw = (uint32_t)(n0 + lcb * 4) * 4u + (uint32_t)rr * (uint32_t)ldb * 4u;
+      b_off[i] = n0 + lcb * 4 < N ? b_raw : 0x80000000u;
+      b_tail[i] = rr < KLAST ? b_raw + (uint32_t)((KT - 1) * BK * 4) * (uint32_t)ldb : 0x80000000u;
     }
     auto dma = [&](int kt) {
       const uint32_t st = lds0 + (uint32_t)((kt % NSTAGE) * STF) * 4u;
@@ -1852,11 +1871,11 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
           eas_dma16s(ra, 0x80000000u, 0u, st + (pw * 4 + i) * 1024);
           eas_dma16s(rb, 0x80000000u, 0u, st + AST * 4 + (pw * 4 + i) * 1024);
         }
-      } else if (K % BK != 0 && kt == KT - 1) {
+      } else if (kt == KT - 1) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          eas_dma16s(ra, a_tail[i], sa, st + (pw * 4 + i) * 1024);
-          eas_dma16s(rb, b_tail[i], sb, st + AST * 4 + (pw * 4 + i) * 1024);
+          eas_dma16s(ra, a_tail[i], 0u, st + (pw * 4 + i) * 1024);
+          eas_dma16s(rb, b_tail[i], 0u, st + AST * 4 + (pw * 4 + i) * 1024);
         }
       } else {
 #pragma unroll
@@ -1941,6 +1960,16 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
     __builtin_amdgcn_sched_group_barrier(0x008, 24, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
+  auto mask_tail = [&](eas_f32x4 (&a)[2][4]) {  // as in the 64 x 64 entry
+    if constexpr (K % 4 != 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[i][u][e] = (KT - 1) * BK + 4 * u + e + 16 * c >= K ? 0.0f : a[i][u][e];
+    }
+  };
   __syncthreads();  // stage 0 landed
   eas_f32x4 a0[2][4], a1[2][4];
   float b0[2][16], b1[2][16];
@@ -1950,8 +1979,10 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
     step(kt, a0, b0, a1, b1);
     step(kt + 1, a1, b1, a0, b0);
   }
+  if constexpr (KT % 2 != 0) mask_tail(a0);
   if constexpr (KT % 2 == 0) {
     step(KT - 2, a0, b0, a1, b1);
+    mask_tail(a1);
     mfmas(a1, b1);
   } else {
     mfmas(a0, b0);
