@@ -36,6 +36,7 @@ M*N below 2^32 (the u32 index range the reference computes in).
 
 from __future__ import annotations
 
+import math
 import os
 
 from dataclasses import dataclass
@@ -147,6 +148,7 @@ class GemmSpec:
     col_base: str | None = None
     col_masked: bool = True       # outputs/operands bounded by col < N (else by the launched grid)
     op_dtype: DType = DType.F16   # MFMA operand type: the dtype of the threadgroup tiles A and B pass through
+    ordered: bool = False         # fp32: each output is the fma chain over ascending k from +0, bit for bit
 
 
 # ---------------------------------------------------------------------------
@@ -961,6 +963,160 @@ def analyze_dot(ir: IRModule, block: int) -> GemmSpec:
 # ---------------------------------------------------------------------------
 # lowering and launch planning
 # ---------------------------------------------------------------------------
+
+
+def analyze_chain(ir: IRModule, block: int) -> GemmSpec:
+    """The matmul with one thread per output (``examples/matmul.py:23-43``): a thread-mode kernel whose
+    threads each store
+
+        C[row*N + col] = fma(A[row*K + K-1], B[(K-1)*N + col], ... fma(A[row*K], B[col], 0.0))
+
+    with row one program id, col = BLOCK * the other + the thread's index, and every access masked
+    by row < M and col < N (a load may leave a bound out: its value then reaches no store).  Proven
+    on the indices as polynomials over the program ids, the thread's index and the u32 scalars.
+    ``plan_gemm`` keeps every index below 2^32, where the kernel's own u32 indices do not wrap.
+    """
+    poly: dict[int, dict[Mono, int]] = {}
+    mask: dict[int, frozenset] = {}
+    load: dict[int, tuple[str, dict[Mono, int], frozenset]] = {}
+    chain: dict[int, tuple[int, int, int] | None] = {}  # None: the constant +0; (previous value, operands)
+    bufs = {a.name: a for a in ir.args if a.kind == "buffer"}
+    name: dict[int, str] = {}
+    stores = []
+    atoms: dict[Any, tuple[dict[Mono, int], dict[Mono, int]]] = {}
+
+    def freeze(p: dict[Mono, int]) -> tuple:
+        return tuple(sorted((m, c) for m, c in p.items() if c))
+
+    for inst in ir.insts:
+        op, out, a = inst.op, inst.out, inst.args
+        if out is not None and out.lanes != 1:
+            raise Unsupported("vector lanes")
+        if op == "arg":
+            name[out.id] = str(a[0])
+            if out.dtype == DType.U32 and a[1] == "scalar":
+                poly[out.id] = {(str(a[0]),): 1}
+        elif op == "const":
+            if out.dtype == DType.U32:
+                poly[out.id] = {(): int(a[0])}
+            elif out.dtype == DType.BOOL and a[0] is True:
+                mask[out.id] = frozenset()
+            elif out.dtype == DType.F32 and float(a[0]) == 0.0 and math.copysign(1.0, float(a[0])) > 0:
+                chain[out.id] = None
+        elif op == "program_id":
+            poly[out.id] = {(f"%pid{int(a[0])}",): 1}
+        elif op == "thread_id":  # program_id(0) * BLOCK + tid, as the thread-id rewrite writes it
+            poly[out.id] = {("%pid0",): block, ("%tid",): 1} if int(a[0]) == 0 else {(f"%pid{int(a[0])}",): 1}
+        elif op == "tid":
+            if int(a[0]) != 0 or int(a[1]) != block:
+                raise Unsupported("thread ids that do not start at 0")
+            poly[out.id] = {("%tid",): 1}
+        elif op in ("add", "mul") and out.dtype == DType.U32:
+            x, y = (poly.get(v.id) for v in a)
+            if x is None or y is None:
+                raise Unsupported("an index that is not a polynomial")
+            r: dict[Mono, int] = {}
+            if op == "add":
+                for p in (x, y):
+                    for m, c in p.items():
+                        r[m] = r.get(m, 0) + c
+            else:
+                for m1, c1 in x.items():
+                    for m2, c2 in y.items():
+                        m = tuple(sorted(m1 + m2))
+                        r[m] = r.get(m, 0) + c1 * c2
+            poly[out.id] = {m: c for m, c in r.items() if c}
+        elif op == "lt" and a[0].dtype == DType.U32:
+            x, y = (poly.get(v.id) for v in a)
+            if x is None or y is None:
+                raise Unsupported("a bound that is not a polynomial")
+            key = (freeze(x), freeze(y))
+            atoms[key] = (x, y)
+            mask[out.id] = frozenset([key])
+        elif op == "and":
+            if any(v.id not in mask for v in a):
+                raise Unsupported("a mask that is not a bound")
+            mask[out.id] = mask[a[0].id] | mask[a[1].id]
+        elif op == "load":
+            if a[0].id not in name or a[2].id not in mask or a[1].id not in poly or out.dtype != DType.F32:
+                raise Unsupported("a load that is not a masked f32 load at a polynomial index")
+            load[out.id] = (name[a[0].id], poly[a[1].id], mask[a[2].id])
+        elif op == "fma":
+            if a[2].id not in chain or a[0].id not in load or a[1].id not in load:
+                raise Unsupported("an fma outside the chain")
+            chain[out.id] = (a[2].id, a[0].id, a[1].id)
+        elif op == "store":
+            stores.append(a)
+        else:
+            raise Unsupported(f"op {op}")
+    if len(stores) != 1:
+        raise Unsupported("not one store")
+    c_ref, c_off, val, c_mask = stores[0]
+    if c_ref.id not in name or c_off.id not in poly or c_mask.id not in mask or not chain.get(val.id):
+        raise Unsupported("the store is not the chain's")
+    steps: list[tuple[int, int]] = []
+    link = chain[val.id]
+    while link is not None:
+        steps.append(link[1:])
+        link = chain[link[0]]
+    steps.reverse()
+    K = len(steps)
+    c_name, c_poly, bounds = name[c_ref.id], poly[c_off.id], mask[c_mask.id]
+    for row_axis in (0, 1):
+        row = {(f"%pid{row_axis}",): 1}
+        col = {(f"%pid{1 - row_axis}",): block, ("%tid",): 1}
+        for key in bounds:
+            if atoms[key][0] == col and len(atoms[key][1]) == 1:
+                (n_mono, n_coef), = atoms[key][1].items()
+                break
+        else:
+            continue
+        m_atoms = [atoms[k][1] for k in bounds if atoms[k][0] == row]
+        if n_coef != 1 or len(n_mono) != 1 or len(bounds) != 2 or len(m_atoms) != 1:
+            continue
+        n_sym = n_mono[0]
+        if len(m_atoms[0]) != 1 or n_sym.startswith("%"):
+            continue
+        (m_mono, m_coef), = m_atoms[0].items()
+        if m_coef != 1 or len(m_mono) != 1 or m_mono[0].startswith("%"):
+            continue
+        if c_poly != {tuple(sorted((n_sym, f"%pid{row_axis}"))): 1, **col}:
+            continue
+        names = set()
+        for k, (x, y) in enumerate(steps):
+            a_want = {(f"%pid{row_axis}",): K, **({(): k} if k else {})}
+            b_want = {**({(n_sym,): k} if k else {}), **col}
+            if (load[x][1], load[y][1]) != (a_want, b_want):
+                x, y = y, x
+            if (load[x][1], load[y][1]) != (a_want, b_want) or not (load[x][2] | load[y][2]) <= bounds:
+                raise Unsupported("a step's operands are not A[row, k] and B[k, col]")
+            names.add((load[x][0], load[y][0]))
+        if len(names) != 1:
+            raise Unsupported("operands from more than one buffer")
+        (a_name, b_name), = names
+        if len({a_name, b_name, c_name}) != 3 or any(bufs[x].dtype != DType.F32 for x in (a_name, b_name, c_name)):
+            raise Unsupported("buffers that are not three f32 ones")
+        return GemmSpec(a=a_name, b=b_name, c=c_name, m_sym=m_mono[0], n_sym=n_sym, K=K, TM=1, TN=block,
+                        row_axis=row_axis, a_dtype=DType.F32, b_dtype=DType.F32, c_dtype=DType.F32, c_f16=False,
+                        f32=True, op_dtype=DType.F32, ordered=True)
+    raise Unsupported("not one thread per output of a matmul")
+
+
+def try_lift_chain(ir: IRModule, block: int) -> Any:
+    """The ordered fp32 GEMM (entry points ``<name>__mm``) of a one-thread-per-output matmul, else
+    ``None``.  It is added to the kernel's own lowering, which keeps every launch the GEMM's plan
+    does not take (a thread count instead of a grid, indices past 2^32)."""
+    if os.environ.get("EAS_HIP_DISABLE_GEMM_LIFT", "") not in ("", "0"):
+        return None
+    if not any(i.op == "fma" for i in ir.insts):
+        return None
+    try:
+        spec = analyze_chain(ir, block)
+    except Unsupported:
+        return None
+    from .gemm_kernels import emit_gemm
+
+    return emit_gemm(ir, block, spec, name=f"{ir.name}__mm")
 
 
 def try_lift(ir: IRModule, block: int) -> Any:

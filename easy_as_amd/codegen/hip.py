@@ -35,7 +35,7 @@ from __future__ import annotations
 
 import math
 import os
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 from typing import Any, Iterable
 
 from ..ir import DType, IRModule, Inst, ValueRef
@@ -55,6 +55,8 @@ class Geometry:
     workgroups (then ``ppw`` is 1).
     kind ``thread``: logical = threadgroups of ``block_size`` threads (or a 1-D
     thread count); hidden arg = number of live threads along x.
+    A thread kernel's ``params["gemm"]`` is the geometry of the GEMM that computes the same for a
+    launch by whole threadgroups.
     kind ``gemm``: a lifted matmul; ``params`` describe its own tiling.
     """
 
@@ -1067,7 +1069,8 @@ def launch_marker(ir: IRModule, geo: Geometry) -> str:
     ppw = geo.programs_per_wg * geo.unroll if geo.kind in ("spmd", "thread") else 1
     line = (f"// eas-launch: kind={geo.kind} block={geo.block_size} wg={geo.wg_size} ppw={ppw} "
             f"split={geo.split} args={kernarg_bytes(ir)} hidden={hidden}\n")
-    return line + gemm_marker(ir, geo) if geo.kind == "gemm" else line
+    gemm = geo if geo.kind == "gemm" else geo.params.get("gemm")
+    return line + gemm_marker(ir, gemm) if gemm is not None else line
 
 
 def ir_to_hip(ir: IRModule) -> Lowered:
@@ -1077,7 +1080,7 @@ def ir_to_hip(ir: IRModule) -> Lowered:
     if mode == "spmd":
         low = _SpmdEmitter(ir, block).emit()
     else:
-        from .gemm_lift import try_lift
+        from .gemm_lift import try_lift, try_lift_chain
         from .thread_lanes import as_lanes
 
         low = try_lift(ir, block)
@@ -1085,4 +1088,8 @@ def ir_to_hip(ir: IRModule) -> Lowered:
             lanes = as_lanes(ir, block)
             low = _SpmdEmitter(lanes, block, thread_mode=True).emit() if lanes is not None else \
                 _ThreadEmitter(ir, block).emit()
+            mm = try_lift_chain(ir, block)
+            if mm is not None:  # the same source, launch shape and entry, with the GEMM's entries after it
+                geo = replace(low.geometry, params={**low.geometry.params, "gemm": mm.geometry})
+                low = Lowered(low.src + mm.src.replace(PRELUDE, "", 1), low.block_size, low.launch_mode, geo)
     return Lowered(launch_marker(ir, low.geometry) + low.src, low.block_size, low.launch_mode, low.geometry)

@@ -613,7 +613,7 @@ int eas_hip_gemm_shape_parse(const char* src, eas_hip_gemm_shape* out) {
 
 int eas_hip_kernel_set_gemm(eas_hip_kernel* k, const eas_hip_gemm_shape* g) {
   if (!k) return fail(EAS_HIP_ERR_INVALID, "kernel must not be NULL");
-  if (k->shape.kind != EAS_HIP_KIND_GEMM)
+  if (k->shape.kind != EAS_HIP_KIND_GEMM && k->shape.kind != EAS_HIP_KIND_THREAD)
     return fail(EAS_HIP_ERR_INVALID, "the kernel's launch shape is not a lifted GEMM's (set its eas-launch shape first)");
   int rc = check_gemm(g);
   if (rc) return rc;
@@ -703,7 +703,8 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g
                       const uint32_t tptg[3], int compute_units, const char* choice, eas_hip_gemm_plan* out) {
   int rc = check_shape(s);
   if (rc) return rc;
-  if (s->kind != EAS_HIP_KIND_GEMM) return fail(EAS_HIP_ERR_INVALID, "the kernel is not a lifted GEMM");
+  if (s->kind != EAS_HIP_KIND_GEMM && s->kind != EAS_HIP_KIND_THREAD)
+    return fail(EAS_HIP_ERR_INVALID, "the kernel is not a lifted GEMM");
   rc = check_gemm(g);
   if (rc) return rc;
   if (!size || !tptg || !out) return fail(EAS_HIP_ERR_INVALID, "size/tptg/out must not be NULL");
@@ -926,28 +927,37 @@ static int launch_reference(const eas_hip_kernel* k, const void* kernarg, size_t
                 kernarg_size, k->shape.arg_bytes);
   if (kernarg_size && !kernarg) return fail(EAS_HIP_ERR_INVALID, "kernarg is NULL with nonzero size");
   uint32_t grid[3], block[3], hidden[EAS_HIP_MAX_HIDDEN];
+  uint32_t nhidden = k->shape.hidden;
   hipFunction_t fn = k->function;
-  if (k->shape.kind == EAS_HIP_KIND_GEMM) {
-    if (!k->has_gemm)
-      return fail(EAS_HIP_ERR_INVALID, "this lifted GEMM kernel has no GEMM shape attached (eas_hip_kernel_set_gemm "
-                                       "with its source's eas-gemm line)");
+  const bool gemm = k->shape.kind == EAS_HIP_KIND_GEMM;
+  if (gemm && !k->has_gemm)
+    return fail(EAS_HIP_ERR_INVALID, "this lifted GEMM kernel has no GEMM shape attached (eas_hip_kernel_set_gemm "
+                                     "with its source's eas-gemm line)");
+  // a thread kernel with a GEMM beside it runs as the GEMM where its plan takes the launch
+  bool planned = false;
+  if (k->has_gemm) {
     eas_hip_gemm_plan plan;
     int rc = eas_hip_plan_gemm(&k->shape, &k->gemm, kernarg, kernarg_size, arg_bytes, nargs, by_groups, size,
                                tptg ? tptg : kAuto, k->compute_units, nullptr, &plan);
-    if (rc) return rc;
-    if (!plan.launch) return EAS_HIP_OK;
-    memcpy(grid, plan.grid, sizeof(grid));
-    memcpy(block, plan.block, sizeof(block));
-    memcpy(hidden, plan.hidden, sizeof(plan.hidden));
-    fn = k->gemm_fn[plan.entry];
-  } else {
+    if (rc && gemm) return rc;
+    if (!rc) {
+      if (!plan.launch) return EAS_HIP_OK;
+      memcpy(grid, plan.grid, sizeof(grid));
+      memcpy(block, plan.block, sizeof(block));
+      memcpy(hidden, plan.hidden, sizeof(plan.hidden));
+      nhidden = sizeof(plan.hidden) / sizeof(plan.hidden[0]);
+      fn = k->gemm_fn[plan.entry];
+      planned = true;
+    }
+  }
+  if (!planned) {
     int rc = eas_hip_plan_dispatch(&k->shape, by_groups, size, tptg ? tptg : kAuto, grid, block, hidden,
                                    EAS_HIP_MAX_HIDDEN);
     if (rc) return rc;
   }
-  std::vector<uint8_t> blob((kernarg_size + 3) / 4 * 4 + 4 * k->shape.hidden, 0);
+  std::vector<uint8_t> blob((kernarg_size + 3) / 4 * 4 + 4 * nhidden, 0);
   if (kernarg_size) memcpy(blob.data(), kernarg, kernarg_size);
-  memcpy(blob.data() + (kernarg_size + 3) / 4 * 4, hidden, 4 * k->shape.hidden);
+  memcpy(blob.data() + (kernarg_size + 3) / 4 * 4, hidden, 4 * nhidden);
   return launch_fn(fn, blob.data(), blob.size(), grid, block, 0, stream, repeat);
 }
 

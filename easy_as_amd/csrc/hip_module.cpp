@@ -428,14 +428,14 @@ PyObject* py_compiler_version(PyObject*, PyObject*) {
 }
 
 // Attach the launch shape on `src`'s eas-launch line to `k` (a source without one leaves the
-// kernel's shape unknown: it then runs only through launch_groups), and a lifted GEMM's
-// plan inputs on its eas-gemm line.
+// kernel's shape unknown: it then runs only through launch_groups), and the plan inputs on its
+// eas-gemm line: a lifted GEMM's, or those of the GEMM beside a thread kernel.
 int attach_shape(eas_hip_kernel* k, const char* src) {
   if (!src || !strstr(src, "// eas-launch:")) return EAS_HIP_OK;
   eas_hip_launch_shape s;
   int rc = eas_hip_launch_shape_parse(src, &s);
   if (!rc) rc = eas_hip_kernel_set_shape(k, &s);
-  if (rc || s.kind != EAS_HIP_KIND_GEMM) return rc;
+  if (rc || (s.kind != EAS_HIP_KIND_GEMM && !strstr(src, "// eas-gemm:"))) return rc;
   eas_hip_gemm_shape g;
   rc = eas_hip_gemm_shape_parse(src, &g);
   return rc ? rc : eas_hip_kernel_set_gemm(k, &g);
@@ -1092,9 +1092,8 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
       if (groups[i] == 0) Py_RETURN_NOTIMPLEMENTED;  // nothing to run: the full path checks the arguments
     }
   }
-  const bool gemm = f->shape.kind == EAS_HIP_KIND_GEMM;
-  uint64_t lengths[64];  // a lifted GEMM's buffer lengths in bytes, by argument
-  if (gemm && n > 64) Py_RETURN_NOTIMPLEMENTED;
+  uint64_t lengths[64];  // of a launch by grid: the buffers' lengths in bytes, by argument (a GEMM's plan checks them)
+  if (by_grid && n > 64) Py_RETURN_NOTIMPLEMENTED;
   uint8_t blob[512];
   const size_t arg_bytes = f->shape.arg_bytes, total = (arg_bytes + 3) / 4 * 4 + 4 * (size_t)f->shape.hidden;
   if (total > sizeof(blob)) Py_RETURN_NOTIMPLEMENTED;
@@ -1124,7 +1123,7 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
       if (PyErr_Occurred()) return nullptr;
       memcpy(blob + a.offset, &ptr, 8);
       last_tensor = obj;
-      if (gemm) {
+      if (by_grid) {
         PyObject* nb = PyObject_GetAttr(obj, g_s_nbytes);
         if (!nb) return nullptr;
         lengths[i] = PyLong_AsUnsignedLongLong(nb);
@@ -1157,6 +1156,7 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
       if (!b) Py_RETURN_NOTIMPLEMENTED;
       const uint64_t ptr = (uint64_t)(uintptr_t)b->ptr;
       memcpy(blob + a.offset, &ptr, 8);
+      lengths[i & 63] = b->nbytes;
       continue;
     }
     if ((PyObject*)Py_TYPE(obj) != a.expect) Py_RETURN_NOTIMPLEMENTED;
@@ -1180,11 +1180,7 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
     }
   }
   if (!by_grid && nval == 0) Py_RETURN_NONE;  // a zero extent launches nothing
-  if (by_grid && !gemm) {
-    static const uint32_t kAuto[3] = {0, 0, 0};
-    int rc = eas_hip_plan_dispatch(&f->shape, 1, groups, kAuto, f->grid, f->block, f->hidden, EAS_HIP_MAX_HIDDEN);
-    if (rc) Py_RETURN_NOTIMPLEMENTED;  // the full path reports the size error
-  } else if (!by_grid && (!f->have_plan || f->plan_n != nval)) {
+  if (!by_grid && (!f->have_plan || f->plan_n != nval)) {
     const uint32_t block = f->shape.block_size;
     const uint64_t size[3] = {f->by_groups ? (nval + block - 1) / block : nval, 1, 1};
     static const uint32_t kAuto[3] = {0, 0, 0};
@@ -1210,7 +1206,7 @@ PyObject* py_fast_call(PyObject*, PyObject* const* argv, Py_ssize_t nargv) {
     if (PyErr_Occurred()) return nullptr;
   }
   int rc;
-  if (gemm) {
+  if (by_grid) {
     rc = eas_hip_launch_threadgroups(f->k, blob, arg_bytes, lengths, (int)n, groups, nullptr, stream, 1);
     if (rc == EAS_HIP_ERR_INVALID) Py_RETURN_NOTIMPLEMENTED;  // refused before a launch: the full path reports it
   } else {

@@ -163,6 +163,18 @@ def plan_launch(
             raise ValueError(f"spmd launch of {groups[0]} programs exceeds 2^32 threads along x")
         return LaunchPlan((nblocks, groups[1], groups[2]), (geo.wg_size, 1, 1), (groups[0],))
     if geo.kind == "thread":
+        gemm = geo.params.get("gemm")
+        if gemm is not None and live_x is None:
+            from ..codegen.gemm_lift import plan_gemm
+
+            try:
+                plan = plan_gemm(gemm, groups, runtime_args, None, compute_units)
+            except (ValueError, KeyError):
+                pass  # a launch the GEMM does not take: the kernel's own threads run it
+            else:
+                if plan is not None:
+                    plan.entry = plan.entry or gemm.entry
+                return plan
         # one workgroup per threadgroup, or (a kernel emitted as lanes) the SPMD mapping of one
         # program per threadgroup; the hidden extent is the live thread count either way
         live = live_x if live_x is not None else groups[0] * block
@@ -247,8 +259,10 @@ class HipRuntime:
         if k is None:
             mod = self._mod()
             if callable(getattr(mod, "compile_to_code", None)) and callable(getattr(mod, "load", None)):
-                # the source's eas-launch line gives the kernel its launch shape and argument size
-                k = mod.load(compile_code(mod, ck.src, main), entry, src=ck.src)
+                # the source's eas-launch line gives the kernel its launch shape and argument size; the
+                # GEMM entries beside a thread kernel take other hidden arguments, which their plan gives
+                gemm = ck.geometry is not None and ck.geometry.kind == "thread" and entry != main
+                k = mod.load(compile_code(mod, ck.src, main), entry, src=None if gemm else ck.src)
             else:
                 k = mod.compile(ck.src, entry)
             self._kernels[key] = k
@@ -474,11 +488,11 @@ class HipRuntime:
               shape: Any) -> tuple[LaunchPlan | None, list[bytes]]:
         """The launch plan and its packed hidden arguments.  An SPMD or thread-mode plan
         depends only on the kernel, the launch options and the scalars that size the grid
-        (``N``, ``H``, ``W``, ``D``), so it is cached on those; a lifted GEMM's plan also
+        (``N``, ``H``, ``W``, ``D``), so it is cached on those; a plan that may be a GEMM's also
         checks its buffers' sizes and addresses and is made afresh each time."""
         geo = ck.geometry
         key = None
-        if geo is not None and geo.kind != "gemm":
+        if geo is not None and geo.kind != "gemm" and "gemm" not in geo.params:
             key = (id(ck), nthreads, grid, tptg, shape, runtime_args.get("N"), runtime_args.get("H"),
                    runtime_args.get("W"), runtime_args.get("D"))
             try:
