@@ -26,7 +26,7 @@ is 4-byte aligned; each matrix under 2 GiB):
 
 * A and B go HBM -> LDS with ``buffer_load_dwordx4 ... lds`` (no staging
   registers), BK = 32 per stage, a 4-stage ring (128 KB), so loads are issued
-  three stages ahead;
+  three stages ahead (BK = 64 in the smaller-tile entries);
 * LDS holds A as [m][k] and B as [k][n] (the layouts of HBM); 16-byte chunks
   are XOR-swizzled by row so fragment reads are bank-conflict free;
 * A fragments are ``ds_read_b128`` (8 consecutive k per lane); B fragments are
@@ -637,13 +637,19 @@ static __device__ __forceinline__ void eas_gemm_elementwise(const AT* __restrict
 
 // BM x BN tile body (128 x 64, 128 x 128, 128 x 256 or 64 x 64) for launches whose 256 x 256 grid
 // would leave CUs idle: 8 waves (512 threads), specialised like the fp32 entries, on a ring of 4
-// stages of BM / 16 KB of A and BN / 16 KB of B.  Waves 4-7 produce: the DMA of stage kt+3,
-// BM / 64 A + BN / 64 B loads of 1 KB per wave per stage, with the stage offset in soffset, so the
-// loads cost the MFMA waves sharing their SIMDs nothing.  Waves 0-3 consume, BM/2 x BN/2 each
+// stages (3 of 128 x 256) of BM / 8 KB of A and BN / 8 KB of B.  Waves 4-7 produce: BM / 32 A +
+// BN / 32 B loads of 1 KB per wave per stage, with the stage offset in soffset, so the loads cost
+// the MFMA waves sharing their SIMDs nothing.  Waves 0-3 consume, BM/2 x BN/2 each, in halves of 32 k
 // (MI 16: BM/32 x BN/32 accumulators of 16x16x32; MI 32: 2 x BN/64 of 32x32x16): the fragments of
-// stage kt+1 are read between stage kt's MFMAs.  A load costs the SIMD that issues it tens of clocks of MFMA issue, which in a
-// 4-wave form of this body (each wave loading its quarter of every stage beside its MFMAs) was
-// most of the stage.
+// one half are read between the MFMAs of the half before.  A load costs the SIMD that issues it
+// tens of clocks of MFMA issue, which in a 4-wave form of this body (each wave loading its quarter
+// of every stage beside its MFMAs) was most of the stage.
+//
+// BK = 64, because a CU takes lines from L2, not bytes: the 64-byte rows of A of a BK = 32 stage run
+// at 66 B/ns where 128-byte ones run at 117 (a read loop on all CUs), and these loops wait on that.
+// Against stages of 32 (and the barrier before each): 1024 x 1024 x 4096 f16 27.7 -> 17.1 us (64 x 64),
+// 2048 x 1024 x 2048 15.5 -> 13.3 (128 x 64), 256 x 14336 x 4096 bf16 39.4 -> 32.0 (128 x 128),
+// 512 x 14336 x 4096 bf16 with B from HBM 79.7 -> 64.7 (128 x 256; there MFMA- and HBM-bound in turn).
 template <typename CT, int K, int BN, int MI = 16, int BM = 128>
 static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict__ A, const eas_op_t* __restrict__ B,
                                                      CT* __restrict__ C, int ldb, int M, int N, int m0, int n0,
@@ -651,10 +657,10 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
   static_assert((BN == 64 || BN == 128 || BN == 256) && (MI == 32 || MI == 16) && (BN != 64 || MI == 16) &&
                     (BM == 128 || (BM == 64 && BN == 64)),
                 "128 x 64, 128 x 128, 128 x 256 or 64 x 64 tiles; 32- or 16-row MFMAs (16 on 64 columns)");
-  constexpr int BK = 32, NSTAGE = 4, KT = (K + BK - 1) / BK;
-  constexpr int NAI = BM / 64;              // A loads per producer wave per stage (1 or 2)
+  constexpr int BK = 64, NSTAGE = BN == 256 ? 3 : 4, KT = (K + BK - 1) / BK, HT = (K + 31) / 32;  // HT: halves
+  constexpr int NAI = BM / 32;              // A loads per producer wave per stage (2 or 4)
   constexpr int NJ = BN / 64;               // 32-column accumulators per consumer wave
-  constexpr int NBI = BN / 64;              // B loads per producer wave per stage (1, 2 or 4)
+  constexpr int NBI = BN / 32;              // B loads per producer wave per stage (2, 4 or 8)
   constexpr int CH = BN / 8;                // 16-byte chunks per B row
   constexpr int STAGE_A = BM * BK, STAGE_B = BK * BN;  // halves per stage
   constexpr int KLAST = K - (KT - 1) * BK;  // k extent of the last stage
@@ -671,15 +677,16 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
     return BN == 64 ? 2 * ((r >> 1) & 1) + 4 * ((r >> 3) & 1) : (4 * (r & 3)) ^ (2 * ((r >> 3) & 1));
   };
   if (wave >= 4) {
-    // DMA instructions write 1 KB of a stage each.  A instruction q = 2 pw + i: rows 16q + lane/4,
-    // chunk lane%4 stored at chunk ^ ((row/4)%4).  B instruction q = NBI pw + i: rows
+    // DMA instructions write 1 KB of a stage each.  A instruction q = NAI pw + i: rows 8q + lane/8,
+    // chunk lane%8 stored at chunk ^ ((row/2)%8).  B instruction q = NBI pw + i: rows
     // (64 / CH) q + lane / CH, chunk lane % CH stored at chunk ^ bsw(row).
-    // Rows past M load zeros, and so do columns past N when no 8-column chunk straddles N, so
-    // every address a load reads, lane offset plus stage offset, lies inside A or B.  An edge tile
-    // whose chunk straddles N (N % 8 != 0) adds the stage offset to the lane offset instead, where
-    // the range check sees all of it.  The last stage of a K that is not a multiple of BK does the
-    // same (its straddling A chunk may end past A); stages past K load zeros into a slot nobody
-    // reads, so every stage issues the same loads and the count at each barrier is the same.
+    // Rows past M and chunks past N load zeros, and a chunk that straddles N reads on into B's next
+    // row, so in every stage but the last each address a load reads, lane offset plus stage offset,
+    // lies inside A or B (rows of under 8 columns add the stage offset to the lane offset instead).
+    // The last stage keeps the whole offset in the lane, where the range check sees all of it: zeros
+    // past K and past the end of B, but for the A chunk that straddles K, which the consumers mask.
+    // Stages past K load zeros into a slot nobody reads, so every stage issues the same loads and
+    // the count at each barrier is the same.
     const int pw = wave - 4;
     const eas_rsrc ra = eas_make_rsrc(A, (uint32_t)M * (uint32_t)K * 2u);
     const eas_rsrc rb = eas_make_rsrc(B, ((uint32_t)(K - 1) * (uint32_t)ldb + (uint32_t)N) * 2u);
@@ -688,8 +695,8 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
 #pragma unroll
     for (int i = 0; i < NAI; ++i) {
       const int q = pw * NAI + i;
-      const int r_a = 16 * q + (lane >> 2);
-      const int c_a = (lane & 3) ^ ((r_a >> 2) & 3);
+      const int r_a = 8 * q + (lane >> 3);
+      const int c_a = (lane & 7) ^ ((r_a >> 1) & 7);
       const uint32_t a_raw = ((uint32_t)(m0 + r_a) * (uint32_t)K + (uint32_t)(c_a * 8)) * 2u;
       a_off[i] = m0 + r_a < M ? a_raw : 0x80000000u;
       a_tail[i] = (m0 + r_a < M && c_a * 8 < KLAST) ? a_raw + (uint32_t)((KT - 1) * BK * 2) : 0x80000000u;
@@ -703,55 +710,54 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
       b_off[i] = n0 + c_b * 8 < N ? b_raw[i] : 0x80000000u;
       b_tail[i] = r_b < KLAST ? b_raw[i] + (uint32_t)((KT - 1) * BK * 2) * (uint32_t)ldb : 0x80000000u;
     }
-    auto dma = [&](int kt, auto b_fast) {
-      const uint32_t st_a = lds_a + (uint32_t)((kt % NSTAGE) * STAGE_A * 2);
-      const uint32_t st_b = lds_b + (uint32_t)((kt % NSTAGE) * STAGE_B * 2);
+    auto dma = [&](int kt, auto b_fast) __attribute__((always_inline)) {
+      const uint32_t st_a = lds_a + (uint32_t)((kt % NSTAGE) * STAGE_A * 2 + pw * NAI * 1024);
+      const uint32_t st_b = lds_b + (uint32_t)((kt % NSTAGE) * STAGE_B * 2 + pw * NBI * 1024);
       const uint32_t sa = (uint32_t)(kt * BK * 2), sb = (uint32_t)(kt * BK * 2) * (uint32_t)ldb;
+      if (kt >= KT) {
 #pragma unroll
-      for (int i = 0; i < NAI; ++i) {
-        const uint32_t dst = st_a + (uint32_t)((pw * NAI + i) * 1024);
-        if (kt >= KT)
-          eas_dma16s(ra, 0x80000000u, 0u, dst);
-        else if (K % BK != 0 && kt == KT - 1)
-          eas_dma16s(ra, a_tail[i], 0u, dst);
-        else
-          eas_dma16s(ra, a_off[i], sa, dst);
-      }
+        for (int i = 0; i < NAI; ++i) eas_dma16s(ra, 0x80000000u, 0u, st_a + i * 1024);
 #pragma unroll
-      for (int i = 0; i < NBI; ++i) {
-        const uint32_t dst = st_b + (uint32_t)((pw * NBI + i) * 1024);
-        if (kt >= KT)
-          eas_dma16s(rb, 0x80000000u, 0u, dst);
-        else if (K % BK != 0 && kt == KT - 1)
-          eas_dma16s(rb, b_tail[i], 0u, dst);
-        else if constexpr (decltype(b_fast)::value)
-          eas_dma16s(rb, b_off[i], sb, dst);
-        else
-          eas_dma16s(rb, b_raw[i] + sb, 0u, dst);
+        for (int i = 0; i < NBI; ++i) eas_dma16s(rb, 0x80000000u, 0u, st_b + i * 1024);
+      } else if (kt == KT - 1) {
+#pragma unroll
+        for (int i = 0; i < NAI; ++i) eas_dma16s(ra, a_tail[i], 0u, st_a + i * 1024);
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) eas_dma16s(rb, b_tail[i], 0u, st_b + i * 1024);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NAI; ++i) eas_dma16s(ra, a_off[i], sa, st_a + i * 1024);
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+          if constexpr (decltype(b_fast)::value)
+            eas_dma16s(rb, b_off[i], sb, st_b + i * 1024);
+          else
+            eas_dma16s(rb, b_raw[i] + sb, 0u, st_b + i * 1024);
+        }
       }
     };
     // one barrier per stage, as many as the consumers
-    auto produce = [&](auto b_fast) {
+    auto produce = [&](auto b_fast) __attribute__((always_inline)) {
       constexpr int PER = NAI + NBI;  // loads per stage
 #pragma unroll
-      for (int p = 0; p < NSTAGE - 1; ++p) dma(p, b_fast);
-      __builtin_amdgcn_s_waitcnt(EAS_WAITVM(2 * PER));  // stage 0 landed (stages 1 and 2 may be in flight)
+      for (int p = 0; p < NSTAGE; ++p) dma(p, b_fast);
+      __builtin_amdgcn_s_waitcnt(EAS_WAITVM((NSTAGE - 1) * PER));  // stage 0 landed
       __syncthreads();
       for (int kt = 0; kt + 1 < KT; ++kt) {
-        __builtin_amdgcn_s_waitcnt(EAS_WAITVM(PER));  // stage kt+1 landed (stage kt+2 may be in flight)
+        __builtin_amdgcn_s_waitcnt(EAS_WAITVM((NSTAGE - 2) * PER));  // stage kt+1 landed
         __syncthreads();
-        dma(kt + NSTAGE - 1, b_fast);  // the slot of stage kt-1, whose fragments every consumer has read
+        dma(kt + NSTAGE, b_fast);  // the slot of stage kt, whose fragments every consumer has read
       }
       __builtin_amdgcn_s_waitcnt(EAS_WAITVM(0));
     };
-    if (n0 + BN <= N || N % 8 == 0)
+    if (n0 + BN <= N || N % 8 == 0 || ldb >= 8)
       produce(eas_bool_c<true>{});
     else
       produce(eas_bool_c<false>{});
     return;
   }
   const int wm = wave >> 1, wn = wave & 1;
-  // Fragments per stage: 4 of A and BN / 32 of B, 8 halves a lane each.  MI 32
+  // Fragments per half (32 k): 4 of A and BN / 32 of B, 8 halves a lane each.  MI 32
   // (v_mfma_f32_32x32x16): A f = 2 ks + i holds A[row 32 i + l%32][k 16 ks + 8(l/32)..+7], B f =
   // ks NJ + j holds B[k 16 ks + 8(l/32)..+7][col 32 j + l%32]; MI 16 (v_mfma_f32_16x16x32): A f = i
   // holds A[row 16 i + l%16][k 8(l/16)..+7], B f = j holds B[k 8(l/16)..+7][col 16 j + l%16]
@@ -762,7 +768,7 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
   for (int f = 0; f < NA; ++f) {
     const int r = MI == 32 ? wm * 64 + (f & 1) * 32 + (lane & 31) : wm * (BM / 2) + f * 16 + (lane & 15);
     const int c = MI == 32 ? (2 * (f >> 1) + (lane >> 5)) : (lane >> 4);
-    fa_off[f] = r * BK + ((c ^ ((r >> 2) & 3)) * 8);
+    fa_off[f] = r * BK + ((c ^ ((r >> 1) & 7)) * 8);  // the second half's chunks are 4 on: offset ^ 32
   }
 #pragma unroll
   for (int f = 0; f < NB; ++f) {
@@ -786,11 +792,12 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
     for (int j = 0; j < NB; ++j) acc16[i][j] = (eas_f32x4){};
   typedef eas_h8 afrag_t[NA];
   typedef eas_h8 bfrag_t[NB];
-  auto read_stage = [&](int kt, afrag_t& fa, bfrag_t& fb) {
-    const eas_op_t* as = As + (kt % NSTAGE) * STAGE_A;
-    const eas_op_t* bs = Bs + (kt % NSTAGE) * STAGE_B;
+  auto read_half = [&](int h, afrag_t& fa, bfrag_t& fb) {
+    const int hb = h & 1;
+    const eas_op_t* as = As + (h / 2 % NSTAGE) * STAGE_A;
+    const eas_op_t* bs = Bs + (h / 2 % NSTAGE) * STAGE_B + hb * 32 * BN;
 #pragma unroll
-    for (int f = 0; f < NA; ++f) fa[f] = *(const eas_h8*)(as + fa_off[f]);
+    for (int f = 0; f < NA; ++f) fa[f] = *(const eas_h8*)(as + (fa_off[f] ^ (32 * hb)));
 #pragma unroll
     for (int f = 0; f < NB; ++f) {
       const eas_h4t lo = EAS_DS_TR16((EAS_LDS eas_h4t*)(bs + fb_off[f]));
@@ -814,15 +821,15 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
         for (int j = 0; j < NB; ++j) acc16[i][j] = EAS_MFMA16(fa[i], fb[j], acc16[i][j], 0, 0, 0);
     }
   };
-  // At the barrier of stage kt the producers' DMA of stage kt+1 has landed; after it the wave
-  // issues stage kt's MFMAs from the fragments read one stage earlier and, between them, every
-  // fragment read of stage kt+1 into the other set.  After this barrier the producers refill the
-  // slot of stage kt-1, whose fragments every consumer read (and used) before it.
-  auto step = [&](int kt, const afrag_t& fa, const bfrag_t& fb, afrag_t& na, bfrag_t& nb) {
+  // Half h: its MFMAs, from the fragments read during the half before, and between them every fragment
+  // read of half h+1 into the other set.  Before the second half of a stage: the barrier at which
+  // the next stage has landed, and after which the producers refill this stage's slot, both of
+  // whose halves every consumer has read (and waited for) before it.
+  auto step = [&](int h, const afrag_t& fa, const bfrag_t& fb, afrag_t& na, bfrag_t& nb) {
     constexpr int NMFMA = MI == 32 ? 4 * NJ : NA * NB, NREAD = NA + 2 * NB;
-    __syncthreads();
+    if (h & 1) __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    read_stage(kt + 1, na, nb);
+    read_half(h + 1, na, nb);
     mfmas(fa, fb);
 #pragma unroll
     for (int s = 0; s < NREAD / 2; ++s) {  // the LDS reads two by two after the first MFMAs
@@ -832,14 +839,14 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
     __builtin_amdgcn_sched_group_barrier(0x008, NMFMA - NREAD / 2, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
-  // the last stage of a K that is not a multiple of 8: halves at k >= K hold the next row of A
+  // the last half of a K that is not a multiple of 8: elements at k >= K hold the next row of A
   auto mask_tail = [&](afrag_t& fa) {
     if constexpr (K % 8 != 0) {
 #pragma unroll
       for (int f = 0; f < NA; ++f)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int k = (KT - 1) * BK + (MI == 32 ? 16 * (f >> 1) + 8 * (lane >> 5) : 8 * (lane >> 4)) + e;
+          const int k = (HT - 1) * 32 + (MI == 32 ? 16 * (f >> 1) + 8 * (lane >> 5) : 8 * (lane >> 4)) + e;
           fa[f][e] = k >= K ? (eas_op_t)0.0f : fa[f][e];
         }
     }
@@ -847,14 +854,13 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
   __syncthreads();  // stage 0 landed
   afrag_t a0, a1;
   bfrag_t b0, b1;
-  read_stage(0, a0, b0);
-  int kt = 0;
-  for (; kt + 2 < KT; kt += 2) {  // two stages per iteration: the fragment sets alternate
-    step(kt, a0, b0, a1, b1);
-    step(kt + 1, a1, b1, a0, b0);
+  read_half(0, a0, b0);
+  for (int h = 0; h + 2 < HT; h += 2) {  // one stage per iteration: the fragment sets alternate
+    step(h, a0, b0, a1, b1);
+    step(h + 1, a1, b1, a0, b0);
   }
-  if constexpr (KT % 2 == 0) {
-    step(KT - 2, a0, b0, a1, b1);
+  if constexpr (HT % 2 == 0) {
+    step(HT - 2, a0, b0, a1, b1);
     mask_tail(a1);
     mfmas(a1, b1);
   } else {
@@ -1512,7 +1518,7 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128(
   const BT* __restrict__ B = @B@ + __eas_n_lo;
   CT* __restrict__ C = @C@ + (size_t)__eas_m_lo * ldb + __eas_n_lo;
   const int M = (int)(__eas_m_hi - __eas_m_lo), N = (int)(__eas_n_hi - __eas_n_lo);
-  __shared__ __attribute__((aligned(1024))) eas_op_t smem[2 * 4 * 128 * 32];  // DMA ring 4 x 2 x 8 KB
+  __shared__ __attribute__((aligned(1024))) eas_op_t smem[2 * 4 * 128 * 64];  // DMA ring 4 x 2 x 16 KB
   const bool dma_ok = (K % 2 == 0) && (ldb % 2 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) &&
                       ((uint64_t)M * K * 2 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 2 < (1ull << 31));
   int m0, n0;
@@ -1535,7 +1541,7 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128x256(
   const BT* __restrict__ B = @B@ + __eas_n_lo;
   CT* __restrict__ C = @C@ + (size_t)__eas_m_lo * ldb + __eas_n_lo;
   const int M = (int)(__eas_m_hi - __eas_m_lo), N = (int)(__eas_n_hi - __eas_n_lo);
-  __shared__ __attribute__((aligned(1024))) eas_op_t smem[4 * (128 * 32 + 32 * 256)];  // DMA ring 4 x (8 + 16) KB
+  __shared__ __attribute__((aligned(1024))) eas_op_t smem[3 * (128 * 64 + 64 * 256)];  // DMA ring 3 x (16 + 32) KB
   const bool dma_ok = (K % 2 == 0) && (ldb % 2 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) &&
                       ((uint64_t)M * K * 2 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 2 < (1ull << 31));
   int m0, n0;
@@ -1558,7 +1564,7 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t128x64(
   const BT* __restrict__ B = @B@ + __eas_n_lo;
   CT* __restrict__ C = @C@ + (size_t)__eas_m_lo * ldb + __eas_n_lo;
   const int M = (int)(__eas_m_hi - __eas_m_lo), N = (int)(__eas_n_hi - __eas_n_lo);
-  __shared__ __attribute__((aligned(1024))) eas_op_t smem[4 * (128 * 32 + 32 * 64)];  // DMA ring 4 x (8 + 4) KB
+  __shared__ __attribute__((aligned(1024))) eas_op_t smem[4 * (128 * 64 + 64 * 64)];  // DMA ring 4 x (16 + 8) KB
   const bool dma_ok = (K % 2 == 0) && (ldb % 2 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) &&
                       ((uint64_t)M * K * 2 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 2 < (1ull << 31));
   int m0, n0;
@@ -1581,7 +1587,7 @@ extern "C" __global__ __launch_bounds__(512) void @NAME@__t64x64(
   const BT* __restrict__ B = @B@ + __eas_n_lo;
   CT* __restrict__ C = @C@ + (size_t)__eas_m_lo * ldb + __eas_n_lo;
   const int M = (int)(__eas_m_hi - __eas_m_lo), N = (int)(__eas_n_hi - __eas_n_lo);
-  __shared__ __attribute__((aligned(1024))) eas_op_t smem[4 * (64 * 32 + 32 * 64)];  // DMA ring 4 x (4 + 4) KB
+  __shared__ __attribute__((aligned(1024))) eas_op_t smem[4 * (64 * 64 + 64 * 64)];  // DMA ring 4 x (8 + 8) KB
   const bool dma_ok = (K % 2 == 0) && (ldb % 2 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) &&
                       ((uint64_t)M * K * 2 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 2 < (1ull << 31));
   int m0, n0;
