@@ -91,6 +91,10 @@ template <bool V>
 struct eas_bool_c {  // a compile-time flag passed as a value (to select a loop version)
   static constexpr bool value = V;
 };
+template <int V>
+struct eas_int_c {
+  static constexpr int value = V;
+};
 // 16 bytes per lane, HBM -> LDS; lane i writes LDS bytes [lds + 16 i, lds + 16 i + 16).
 // Issued as asm so the compiler does not add vmcnt(0) before every LDS read; the
 // pipelines count their own loads with EAS_WAITVM.
@@ -1027,8 +1031,8 @@ static __device__ __forceinline__ void eas_gemm_skinny_dma(const eas_op_t* __res
 // from n0, the four waves split K as above, each moving its range global -> registers -> LDS, R
 // stages of 32 k in flight in registers.  A wave's LDS accesses run in order, so its private slot
 // needs no barrier.  Bound by the rows of B from HBM where the grid fills the chip, else by the latency of
-// a wave's chain of stages.  f16 16 x 14336 x 4097: 18.6 us, 6.3 TB/s; f32 16 x 14336 x 4096: 34.1 us,
-// 6.9 TB/s.  More stages in flight (4, 6) take AGPRs and moves between them: 20.3 and 20.8 us.
+// a wave's chain of stages.  With B in the memory-side cache f16 16 x 14336 x 4097 takes 19.6 us, 6.0
+// TB/s, f32 16 x 14336 x 4096 36.1 us, 6.5 TB/s; from HBM 26.4 and 44.2.
 template <typename AT, typename BT, typename CT, int K, int MT>
 static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict__ A, const BT* __restrict__ B,
                                                             CT* __restrict__ C, int ldb, int M, int N, int n0,
@@ -1038,7 +1042,7 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
   constexpr int UA = eas_unit<AT>(), UB = eas_unit<BT>();
   constexpr int ACH = KS / UA, BCH = NT / UB;                  // units per row of A (within a stage) and of B
   constexpr int NA = MR * ACH / 64, NB = KS * BCH / 64;        // units per lane and stage
-  constexpr int R = NA + NB <= 6 ? 2 : 1;                      // stages in flight
+  constexpr int R = MT == 8 ? 1 : 2;                           // stages in flight
   constexpr int STH = KS * NT + MR * KS;                       // halves: B [32][64], A [MR][32]
   const int tid = eas_tid(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1070,8 +1074,9 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
     return k >= K ? UB : k == K - 1 ? eas_unit_lost<BT>(bn, N) : 0;
   };
   eas_u32x4 ra[R][NA], rb[R][NB];
-  auto load = [&](int t, eas_u32x4 (&xa)[NA], eas_u32x4 (&xb)[NB]) {
-    if (kb + (t + 1) * KS < K) {
+  // steady: a step that lies below K
+  auto load = [&](int t, eas_u32x4 (&xa)[NA], eas_u32x4 (&xb)[NB], auto steady) __attribute__((always_inline)) {
+    if (decltype(steady)::value || kb + (t + 1) * KS < K) {
 #pragma unroll
       for (int i = 0; i < NB; ++i) xb[i] = eas_load_unit(pb[i] + (size_t)t * KS * ldb);
 #pragma unroll
@@ -1103,8 +1108,8 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[mt][j] = (eas_f32x4){};
-  auto step = [&](int t, eas_u32x4 (&xa)[NA], eas_u32x4 (&xb)[NB]) {
-    if (kb + (t + 1) * KS >= K) {
+  auto step = [&](int t, eas_u32x4 (&xa)[NA], eas_u32x4 (&xb)[NB], auto steady) __attribute__((always_inline)) {
+    if (!decltype(steady)::value && kb + (t + 1) * KS >= K) {
 #pragma unroll
       for (int i = 0; i < NB; ++i) xb[i] = eas_unit_end<BT>(xb[i], lost_b(t, i));
 #pragma unroll
@@ -1114,7 +1119,7 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
     for (int i = 0; i < NB; ++i) eas_store_unit<BT>(bs + lb[i], xb[i]);
 #pragma unroll
     for (int i = 0; i < NA; ++i) eas_store_unit<AT>(as + la[i], xa[i]);
-    if (t + R < nsteps) load(t + R, xa, xb);
+    if (decltype(steady)::value || t + R < nsteps) load(t + R, xa, xb, steady);
     eas_h8 a[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) a[mt] = *(const eas_h8*)(as + mt * 16 * KS + fa);
@@ -1130,11 +1135,19 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
   };
 #pragma unroll
   for (int p = 0; p < R; ++p)
-    if (p < nsteps) load(p, ra[p], rb[p]);
-  for (int t = 0; t < nsteps; t += R)
+    if (p < nsteps) load(p, ra[p], rb[p], eas_bool_c<false>{});
+  // without a branch while the step R on is not the last one (a branch would make the compiler wait
+  // for every load in flight at its join)
+  int t = 0;
+#pragma unroll 1
+  for (; t + 2 * R < nsteps; t += R)
+#pragma unroll
+    for (int p = 0; p < R; ++p) step(t + p, ra[p], rb[p], eas_bool_c<true>{});
+#pragma unroll 1
+  for (; t < nsteps; t += R)
 #pragma unroll
     for (int p = 0; p < R; ++p)
-      if (t + p < nsteps) step(t + p, ra[p], rb[p]);
+      if (t + p < nsteps) step(t + p, ra[p], rb[p], eas_bool_c<false>{});
   // every load has been used: said here, so that the compiler does not take them for pending in the
   // entry's other bodies and wait between their DMA loads (decode launches ran 3-8 us longer)
   __builtin_amdgcn_s_waitcnt(EAS_WAITVM(0));
@@ -1170,12 +1183,11 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
 // One barrier per stage, in its middle.  Before it: the MFMAs of the first k half, the reads of
 // the second half's fragments, the stores of stage kt+1 into the other slot (last read before the
 // previous barrier) and the loads of stage kt+2 into the registers this frees.  After it: the MFMAs
-// of the second half and the reads of stage kt+1's first fragments.A second stage
-// in flight needs registers past 256, which cost moves from and to AGPRs: 1024 x 2048 x 2048 f32 on 128 x 64
-// tiles 27.1 us with one stage, 36.5 with two.  Bound by the rate a CU takes lines from L2: a 16-byte
-// load off a 16-byte boundary takes two passes (59 B/ns against 117 aligned in a read loop), so a 128 x 128 x
-// 64 stage of odd rows is about 0.55 us of loads for 0.24 us of MFMAs; 1531 x 2047 x 1023 f16 runs 16.6 us
-// (with the element-wise body this replaces 125.8), 4095^3 140 us = 978 TFLOP/s.
+// of the second half and the reads of stage kt+1's first fragments.Bound by one wave a
+// SIMD doing all of it in turn: without the loads 1531 x 2047 x 1023 f16 takes 13.9 us, without the MFMAs
+// 15.3, and the loads alone about 9 (off a 16-byte boundary each takes two passes: 59 B/ns a CU against
+// 117 aligned, in a read loop).  It runs 16.3 us (on the element-wise body this replaces 125.8), 1024 x
+// 2048 x 2048 f32 22.2 (140.6), 4095^3 f16 140 us = 978 TFLOP/s.
 template <typename AT, typename BT, typename CT, int K, int BM, int BN>
 static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, const BT* __restrict__ B,
                                                      CT* __restrict__ C, int ldb, int M, int N, int m0, int n0,
@@ -1222,16 +1234,16 @@ static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, c
     return k >= K ? UB : k == K - 1 ? eas_unit_lost<BT>(bn, N) : 0;
   };
   eas_u32x4 xa[NA], xb[NB];  // the units of one stage
-  auto load_a = [&](int kt, int i) {
-    if (kt < KT - 1) {
+  auto load_a = [&](int kt, int i, auto last) {
+    if constexpr (!decltype(last)::value) {
       xa[i] = eas_load_unit(pa[i] + (size_t)kt * BK);
     } else {
       const int lost = lost_a();
       xa[i] = eas_load_unit(lost == UA ? A : pa[i] + (size_t)kt * BK - lost);
     }
   };
-  auto load_b = [&](int kt, int i) {
-    if (kt < KT - 1) {
+  auto load_b = [&](int kt, int i, auto last) {
+    if constexpr (!decltype(last)::value) {
       xb[i] = eas_load_unit(pb[i] + (size_t)kt * BK * ldb);
     } else {
       const int lost = lost_b(i);
@@ -1290,11 +1302,15 @@ static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, c
       else acc16[i][j] = EAS_MFMA16(fa[ks][i], fb[ks][j], acc16[i][j], 0, 0, 0);
     }
   };
-  // stage kt, whose first fragments are in registers; xa, xb: stage kt+1's units, then kt+2's
-  auto stage = [&](int kt) {
-    const int s = kt & 1, sn = s ^ 1;
-    const bool next = kt + 1 < KT, more = kt + 2 < KT;
-    if (kt + 1 == KT - 1) finish();
+  // stage kt in slot s, whose first fragments are in registers; xa, xb: stage kt+1's units, then kt+2's.
+  // left: the stages after it, 3 standing for any more (a branch in the loop would make the compiler
+  // wait for every load in flight at its join: in a loop, 1531 x 2047 x 1023 f16 ran 33.3 us instead of 17.1)
+  auto stage = [&](int kt, int s, auto left) __attribute__((always_inline)) {
+    constexpr int LEFT = decltype(left)::value;
+    constexpr bool next = LEFT > 0, more = LEFT > 1;
+    typedef eas_bool_c<LEFT == 2> last_t;
+    const int sn = s ^ 1;
+    if (LEFT == 1) finish();
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
       __builtin_amdgcn_sched_barrier(0);
@@ -1306,12 +1322,12 @@ static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, c
 #pragma unroll
         for (int u = i * NA / TI; u < (i + 1) * NA / TI; ++u) {
           put_a(sn, u);
-          if (more) load_a(kt + 2, u);
+          if (more) load_a(kt + 2, u, last_t{});
         }
 #pragma unroll
         for (int u = i * NB / TI; u < (i + 1) * NB / TI; ++u) {
           put_b(sn, u);
-          if (more) load_b(kt + 2, u);
+          if (more) load_b(kt + 2, u, last_t{});
         }
       }
     }
@@ -1330,26 +1346,48 @@ static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, c
     __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
-  for (int i = 0; i < NB; ++i) load_b(0, i);
+  for (int i = 0; i < NB; ++i) load_b(0, i, eas_bool_c<KT == 1>{});
 #pragma unroll
-  for (int i = 0; i < NA; ++i) load_a(0, i);
+  for (int i = 0; i < NA; ++i) load_a(0, i, eas_bool_c<KT == 1>{});
   if (KT == 1) finish();
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     put_b(0, i);
-    if (KT > 1) load_b(1, i);
+    if constexpr (KT > 1) load_b(1, i, eas_bool_c<KT == 2>{});
   }
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
     put_a(0, i);
-    if (KT > 1) load_a(1, i);
+    if constexpr (KT > 1) load_a(1, i, eas_bool_c<KT == 2>{});
   }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < TJ; ++j) read_b(0, 0, j);
 #pragma unroll
   for (int i = 0; i < TI; ++i) read_a(0, 0, i);
-  for (int kt = 0; kt < KT; ++kt) stage(kt);
+  // Four stages an iteration (two of f32): slots are immediates of the LDS accesses, and the
+  // accumulators the compiler moves once an iteration cost less.  Up to 16 stages of 16-bit operands
+  // no loop at all (1531 x 2047 x 1023 f16 16.3 us, 17.1 with it).  256 x 256 has no registers for any.
+  constexpr bool BITS16 = sizeof(AT) == 2 && sizeof(BT) == 2;
+  constexpr int STEADY = KT > 3 ? KT - 3 : 0, FOURS = BM == 256 || !BITS16 ? 0 : STEADY / 4 * 4;
+  constexpr int PAIRS = BM == 256 ? 0 : STEADY / 2 * 2, FLAT = KT <= 16 && BITS16 && BM != 256 ? 4 : 1;
+#pragma unroll FLAT
+  for (int kt = 0; kt < FOURS; kt += 4) {
+    stage(kt, 0, eas_int_c<3>{});
+    stage(kt + 1, 1, eas_int_c<3>{});
+    stage(kt + 2, 0, eas_int_c<3>{});
+    stage(kt + 3, 1, eas_int_c<3>{});
+  }
+#pragma unroll FLAT
+  for (int kt = FOURS; kt < PAIRS; kt += 2) {
+    stage(kt, 0, eas_int_c<3>{});
+    stage(kt + 1, 1, eas_int_c<3>{});
+  }
+#pragma unroll FLAT
+  for (int kt = PAIRS; kt < STEADY; ++kt) stage(kt, kt & 1, eas_int_c<3>{});
+  if constexpr (KT > 2) stage(KT - 3, (KT - 3) & 1, eas_int_c<2>{});
+  if constexpr (KT > 1) stage(KT - 2, (KT - 2) & 1, eas_int_c<1>{});
+  stage(KT - 1, (KT - 1) & 1, eas_int_c<0>{});
   __builtin_amdgcn_s_waitcnt(EAS_WAITVM(0));  // as in eas_gemm_skinny_regs: no load is pending
   const bool full = (m0 + BM <= M) && (n0 + BN <= N);
 #pragma unroll

@@ -1256,9 +1256,10 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
 
 
 # Tiles of the main entry's register body (operands the DMA cannot take) and the relative time of one
-# round of them, one workgroup per CU.  Measured per 64 k, f16 with odd rows (f32 operands in
-# brackets): 64 x 64 0.50 us (0.58), 128 x 64 0.62 (0.78), 128 x 128 0.89 (1.03), 256 x 256 1.7 (2.0-2.4).
-REGISTER_TILES = ((64, 64, 10), (128, 64, 13), (128, 128, 18), (256, 256, 36))
+# round of them, one workgroup per CU.  Measured per 64 k at 2999^3, f16 with odd rows (1024 x 2048 x
+# 2048 f32 in brackets): 64 x 64 0.46 us (0.45), 128 x 64 0.54 (0.64), 128 x 128 0.71 (0.88), 256 x 256
+# 1.7 (2.0).
+REGISTER_TILES = ((64, 64, 10), (128, 64, 12), (128, 128, 16), (256, 256, 37))
 
 
 def _register_tiles(m: int, n: int, cus: int) -> int:

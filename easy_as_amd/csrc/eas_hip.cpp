@@ -685,7 +685,7 @@ uint64_t cdiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 uint64_t register_tiles(uint64_t m, uint64_t n, uint64_t cus) {
   static const struct {
     uint64_t bm, bn, w;  // w: relative time of one round (gemm_lift.REGISTER_TILES holds the measurements)
-  } kTiles[] = {{64, 64, 10}, {128, 64, 13}, {128, 128, 18}, {256, 256, 36}};
+  } kTiles[] = {{64, 64, 10}, {128, 64, 12}, {128, 128, 16}, {256, 256, 37}};
   u128 best = 0;
   uint64_t wgs = 0;
   for (const auto& t : kTiles) {

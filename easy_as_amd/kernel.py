@@ -262,16 +262,15 @@ class Kernel:
 
     def __call__(self, /, *args: Any, **kwargs: Any) -> None:
         key = None
-        if "_grid" in kwargs:
-            if self._call_grid(args, kwargs):
-                return
-        elif self._memo_ok and len(args) == self._n_lead and self._autotune_spec is None:
+        if self._memo_ok and len(args) == self._n_lead and self._autotune_spec is None:
             try:
                 kw = tuple(kwargs.items())
                 fast = self._fast.get(kw)
             except TypeError:  # a keyword value the memo does not key
                 kw = fast = None
             if fast is not None and fast(args) is not NotImplemented:
+                return
+            if "_grid" in kwargs and self._call_grid(args, kwargs):
                 return
             try:
                 key = (kw, tuple(map(_light_key, args)))
@@ -303,8 +302,7 @@ class Kernel:
         earlier call of its shape made one; else the full path, which makes one for the calls after
         it.  False: not such a call, nothing done."""
         grid = kwargs["_grid"]
-        if type(grid) is not tuple or not self._memo_ok or len(args) != self._n_lead \
-                or self._autotune_spec is not None or not kwargs.keys() <= self._grid_kw \
+        if type(grid) is not tuple or not kwargs.keys() <= self._grid_kw \
                 or type(kwargs.get("_tptg", ())) is not tuple:
             return False
         kw = tuple([item for item in kwargs.items() if item[0] != "_grid"])

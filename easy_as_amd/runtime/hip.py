@@ -437,8 +437,8 @@ class HipRuntime:
                              tensor_type, streams, EasTensor)
         call, pending, synchronize = mod.fast_call, self._pending, mod.synchronize
 
-        def launch(*call_args: Any) -> Any:  # the arguments' tuple, and the grid of a launch sized by one
-            p = call(fast, *call_args)
+        def launch(call_args: tuple[Any, ...]) -> Any:
+            p = call(fast, call_args)
             if p is None or p is NotImplemented:
                 return p
             pending.append(p)
@@ -446,7 +446,16 @@ class HipRuntime:
                 synchronize(pending.popleft())
             return None
 
-        return launch
+        def launch_grid(call_args: tuple[Any, ...], grid: tuple[int, ...]) -> Any:
+            p = call(fast, call_args, grid)
+            if p is None or p is NotImplemented:
+                return p
+            pending.append(p)
+            while limit and len(pending) > limit:
+                synchronize(pending.popleft())
+            return None
+
+        return launch if n_index >= 0 else launch_grid
 
     # -- launching ------------------------------------------------------------------
     def run(
