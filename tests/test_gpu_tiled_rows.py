@@ -35,7 +35,7 @@ def test_rows_of_any_length(gpu_runtime, monkeypatch, mnk, entry):
     opts = dict(BM=32, BN=32, BK=32, K=k, NT=256)
     ck = kern.compile(*args, **opts)
     plan = plan_launch(ck, dict(zip((x.name for x in ck.ir.args), args)), grid=grid)
-    assert plan.entry == ("matmul_tiled_kernel__t128" if entry == "tile128" and k % 4 == 0 else None)
+    assert plan.entry == ("matmul_tiled_kernel__t128" if entry == "tile128" and n >= 4 else None)
     kern(*args, **opts, _grid=grid)
     c = tc.cpu().numpy()
     assert (c[m * n:] == -7.0).all()
