@@ -1291,12 +1291,13 @@ def _gemm_entry_choice() -> str:
 def _dma_fits(p: dict, runtime_args: Any, K: int, ldb: int, m: int, n_lo: int, n: int, elem: int = 2) -> bool:
     """Whether the DMA entries take this launch.  16-bit f16/bf16 (``elem`` 2): every row of A and B
     (after the move to the rectangle's origin) 4-byte aligned; fp32 (``elem`` 4, its 128 x 128 entry):
-    rows of B from 4 columns on, K of any value (2047^3 120.1 us on 128 x 128 tiles against 127.0 on
-    64 x 64, 2048 x 2048 x 1021 63.9 against 65.4); each operand's extent under 2 GiB.  Device
-    addresses are known here for torch tensors; numpy inputs are staged into fresh allocations, and
+    rows of B from 4 columns on, K a multiple of 4 or from 256 on (2047^3 120.1 us on 128 x 128 tiles
+    against 127.0 on 64 x 64, 2048 x 2048 x 382 29.0 against 30.3; below, neither is ahead by much:
+    2048 x 2048 x 62 10.9 against 11.6, 4096 x 4096 x 254 78.3 against 75.7, and those stay on 64 x
+    64); each operand's extent under 2 GiB.  Device addresses are known here for torch tensors; numpy inputs are staged into fresh allocations, and
     the entries re-check the addresses they get (a misaligned operand takes their slow element-wise
     guard rather than a wrong result)."""
-    if (K % 2 or ldb % 2 or n_lo % 2) if elem == 2 else ldb < 4:
+    if (K % 2 or ldb % 2 or n_lo % 2) if elem == 2 else (ldb < 4 or (K % 4 and K < 256)):
         return False
     if m * K * elem >= 1 << 31 or ((K - 1) * ldb + n) * elem >= 1 << 31:
         return False

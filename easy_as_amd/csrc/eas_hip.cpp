@@ -669,11 +669,11 @@ int read_arg(const void* kernarg, size_t size, int32_t off, size_t bytes, const 
 }
 
 // Whether the DMA entries take the launch: every row of A and B (after the move to the
-// rectangle's origin) 4-byte aligned for 16-bit operands, ldb from 4 on for fp32; each operand's
-// extent under 2 GiB; A and B 4-byte aligned.
+// rectangle's origin) 4-byte aligned for 16-bit operands; for fp32 ldb from 4 on and K a multiple
+// of 4 or from 256 on; each operand's extent under 2 GiB; A and B 4-byte aligned.
 bool dma_fits(uint64_t a_ptr, uint64_t b_ptr, uint64_t K, uint64_t ldb, uint64_t m, uint64_t n_lo, uint64_t n,
               uint64_t elem) {
-  if (elem == 2 ? (K % 2 || ldb % 2 || n_lo % 2) : ldb < 4) return false;
+  if (elem == 2 ? (K % 2 || ldb % 2 || n_lo % 2) : (ldb < 4 || (K % 4 && K < 256))) return false;
   if ((u128)m * K * elem >= ((u128)1 << 31) || ((u128)(K - 1) * ldb + n) * elem >= ((u128)1 << 31)) return false;
   return a_ptr % 4 == 0 && b_ptr % 4 == 0;
 }

@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("entry", ["auto", "tile128"])
 @pytest.mark.parametrize("mnk", [(1, 1, 1), (3, 5, 3), (65, 67, 31), (64, 66, 33), (130, 129, 62), (129, 131, 64),
-                                 (70, 333, 127), (257, 63, 130), (33, 259, 771), (200, 301, 100), (128, 126, 2)])
+                                 (70, 333, 127), (257, 63, 130), (33, 259, 771), (200, 301, 100), (128, 126, 2),
+                                 (130, 129, 257), (129, 131, 290), (70, 333, 287), (257, 63, 319)])
 def test_rows_of_any_length(gpu_runtime, monkeypatch, mnk, entry):
     import torch
 
@@ -35,7 +36,7 @@ def test_rows_of_any_length(gpu_runtime, monkeypatch, mnk, entry):
     opts = dict(BM=32, BN=32, BK=32, K=k, NT=256)
     ck = kern.compile(*args, **opts)
     plan = plan_launch(ck, dict(zip((x.name for x in ck.ir.args), args)), grid=grid)
-    assert plan.entry == ("matmul_tiled_kernel__t128" if entry == "tile128" and n >= 4 else None)
+    assert plan.entry == ("matmul_tiled_kernel__t128" if entry == "tile128" and (k % 4 == 0 or k >= 256) else None)
     kern(*args, **opts, _grid=grid)
     c = tc.cpu().numpy()
     assert (c[m * n:] == -7.0).all()
