@@ -1027,7 +1027,7 @@ static __device__ __forceinline__ void eas_gemm_skinny_dma(const eas_op_t* __res
   }
 }
 
-// Skinny path for inputs the DMA cannot take (f32, or rows of A or B not 16-byte aligned): 64 columns
+// Skinny path for inputs the DMA cannot take (f32, odd K, odd ldb, odd addresses): 64 columns
 // from n0, the four waves split K as above, each moving its range global -> registers -> LDS, R
 // stages of 32 k in flight in registers.  A wave's LDS accesses run in order, so its private slot
 // needs no barrier.  Bound by the rows of B from HBM where the grid fills the chip, else by the latency of
@@ -1183,11 +1183,11 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
 // One barrier per stage, in its middle.  Before it: the MFMAs of the first k half, the reads of
 // the second half's fragments, the stores of stage kt+1 into the other slot (last read before the
 // previous barrier) and the loads of stage kt+2 into the registers this frees.  After it: the MFMAs
-// of the second half and the reads of stage kt+1's first fragments.Bound by one wave a
+// of the second half and the reads of stage kt+1's first fragments.  Bound by one wave a
 // SIMD doing all of it in turn: without the loads 1531 x 2047 x 1023 f16 takes 13.9 us, without the MFMAs
 // 15.3, and the loads alone about 9 (off a 16-byte boundary each takes two passes: 59 B/ns a CU against
-// 117 aligned, in a read loop).  It runs 16.3 us (on the element-wise body this replaces 125.8), 1024 x
-// 2048 x 2048 f32 22.2 (140.6), 4095^3 f16 140 us = 978 TFLOP/s.
+// 117 aligned, in a read loop).  It runs 15.8 us (on the element-wise body this replaces 125.8), 1024 x
+// 2048 x 2048 f32 21.6 (140.6), 4095^3 f16 140 us = 978 TFLOP/s.
 template <typename AT, typename BT, typename CT, int K, int BM, int BN>
 static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, const BT* __restrict__ B,
                                                      CT* __restrict__ C, int ldb, int M, int N, int m0, int n0,

@@ -168,10 +168,13 @@ int eas_hip_plan_dispatch(const eas_hip_launch_shape* shape, int by_groups, cons
  * of compute units.  Its source carries a second marker line with what that plan
  * needs (`// eas-gemm: entry=... K=... tm=... ...`): the position of M, N (the row
  * stride of B and C) and the tile-base scalars in the packed arguments, where A, B and
- * C are, the reference's tile per threadgroup and the entry points present.  No
- * counterpart in the reference, whose one pipeline per kernel runs any grid. */
+ * C are, the reference's tile per threadgroup and the entry points present.  A
+ * thread kernel proven to be a matmul with one thread per output carries the line too:
+ * its launches by whole threadgroups run as the GEMM where the plan takes them, any
+ * others as its own threads.  No counterpart in the reference, whose one pipeline per
+ * kernel runs any grid. */
 typedef enum eas_hip_gemm_entry {
-  EAS_HIP_GEMM_MAIN = 0,      /* the kernel's own name: 4 waves (skinny path, register-staged body, fp32 64 x 64) */
+  EAS_HIP_GEMM_MAIN = 0,      /* the kernel's own name: 4 waves (skinny path, register bodies), fp32 64 x 64     */
   EAS_HIP_GEMM_PP = 1,        /* <name>__pp: 8 waves on 256 x 256 tiles                                          */
   EAS_HIP_GEMM_T128 = 2,      /* <name>__t128: 128 x 128 tiles                                                   */
   EAS_HIP_GEMM_T128X256 = 3,  /* <name>__t128x256                                                                 */
@@ -210,8 +213,8 @@ typedef struct eas_hip_gemm_plan {
 /* Parse the `// eas-gemm:` marker line of a lifted GEMM's source.  No GPU needed. */
 int eas_hip_gemm_shape_parse(const char* src, eas_hip_gemm_shape* out);
 
-/* Attach a GEMM shape to a kernel with a GEMM launch shape, resolving every entry
- * point it names in the kernel's code object. */
+/* Attach a GEMM shape to a kernel with a GEMM or thread launch shape, resolving every
+ * entry point it names in the kernel's code object. */
 int eas_hip_kernel_set_gemm(eas_hip_kernel* k, const eas_hip_gemm_shape* gemm);
 
 /* The launch plan of a lifted GEMM for a reference-convention launch, without
