@@ -1237,13 +1237,15 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
     if p.get("pp_entry") and choice != "4wave" and _dma_fits(p, runtime_args, K, ldb, m, n_lo, n):
         # When 256 x 256 tiles would fill at most half of the CUs: 128 x 128 tiles if they take one
         # round of CUs, else 128 x 256 ones (at most twice the 256 x 256 count, so one round too).
-        # If even 128 x 128 would fill at most half of the CUs: 64 x 64 tiles while they need at most
-        # 1.75 rounds of CUs, else 128 x 64 (twice the 128 x 128 count: one round).
+        # If even 128 x 128 would fill at most half of the CUs: 64 x 64 tiles while they take one round
+        # of CUs, else 128 x 64 (twice the 128 x 128 count: one round): us on 128 x 64 and 64 x 64,
+        # 1280^3 10.5 and 11.8 (1.56 rounds), 1792 x 1024 x 4096 23.4 and 30.3 (1.75), 1280 x 1280 x
+        # 512 6.5 and 7.1.  Up to 256 k a call is its launch (5.5 and 5.7) and 64 x 64 may take 1.75.
         small = choice == "auto" and 2 * tiles <= compute_units
         if choice == "tile128x256" or (small and tiles128 > compute_units):
             return LaunchPlan((tiles128x256, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t128x256_entry"])
         tiny = small and 2 * tiles128 <= compute_units
-        if choice == "tile64" or (tiny and 4 * tiles64 <= 7 * compute_units):
+        if choice == "tile64" or (tiny and 4 * tiles64 <= (7 if K <= 256 else 4) * compute_units):
             return LaunchPlan((tiles64, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t64_entry"])
         if choice == "tile128x64" or tiny:
             return LaunchPlan((tiles128x64, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t128x64_entry"])
@@ -1294,9 +1296,9 @@ def _dma_fits(p: dict, runtime_args: Any, K: int, ldb: int, m: int, n_lo: int, n
     rows of B from 4 columns on, K a multiple of 4 or from 256 on (2047^3 120.1 us on 128 x 128 tiles
     against 127.0 on 64 x 64, 2048 x 2048 x 382 29.0 against 30.3; below, neither is ahead by much:
     2048 x 2048 x 62 10.9 against 11.6, 4096 x 4096 x 254 78.3 against 75.7, and those stay on 64 x
-    64); each operand's extent under 2 GiB.  Device addresses are known here for torch tensors; numpy inputs are staged into fresh allocations, and
-    the entries re-check the addresses they get (a misaligned operand takes their slow element-wise
-    guard rather than a wrong result)."""
+    64); each operand's extent under 2 GiB.  Device addresses are known here for torch tensors; numpy
+    inputs are staged into fresh allocations, and the entries re-check the addresses they get (a
+    misaligned operand takes their slow element-wise guard rather than a wrong result)."""
     if (K % 2 or ldb % 2 or n_lo % 2) if elem == 2 else (ldb < 4 or (K % 4 and K < 256)):
         return False
     if m * K * elem >= 1 << 31 or ((K - 1) * ldb + n) * elem >= 1 << 31:

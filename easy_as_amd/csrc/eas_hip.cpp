@@ -806,11 +806,11 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g
   } else if (has(EAS_HIP_GEMM_PP) && ch != k4Wave && fits()) {
     // When 256 x 256 tiles would fill at most half of the CUs: 128 x 128 tiles if they take one
     // round of CUs, else 128 x 256 ones.  If even 128 x 128 would fill at most half of the CUs:
-    // 64 x 64 tiles while they need at most 1.75 rounds of CUs, else 128 x 64.
+    // 64 x 64 tiles while they take one round of CUs (1.75 of up to 256 k), else 128 x 64.
     const bool small = ch == kAuto && 2 * tiles <= cus;
     const bool tiny = small && 2 * tiles128 <= cus;
     if (ch == kTile128x256 || (small && tiles128 > cus)) pick(EAS_HIP_GEMM_T128X256, tiles128x256, g->t128_threads);
-    else if (ch == kTile64 || (tiny && 4 * tiles64 <= 7 * cus)) pick(EAS_HIP_GEMM_T64X64, tiles64, g->t128_threads);
+    else if (ch == kTile64 || (tiny && 4 * tiles64 <= (K <= 256 ? 7 : 4) * cus)) pick(EAS_HIP_GEMM_T64X64, tiles64, g->t128_threads);
     else if (ch == kTile128x64 || tiny) pick(EAS_HIP_GEMM_T128X64, tiles128x64, g->t128_threads);
     else if (ch == kTile128 || small) pick(EAS_HIP_GEMM_T128, tiles128, g->t128_threads);
     else pick(EAS_HIP_GEMM_PP, tiles, g->pp_threads);
