@@ -143,6 +143,14 @@ template <typename T> constexpr int eas_unit() { return 16 / (int)sizeof(T); }
 template <typename T> static __device__ __forceinline__ eas_u32x4 eas_load_unit(const T* p) {
   return *(const eas_u32x4_any*)p;
 }
+// Between a wave's LDS writes and its reads of what other lanes wrote (and before it writes again).  The
+// hardware runs one wave's LDS accesses in order; the compiler keeps only each lane's own order, and may move a
+// read over a write that it proves to be at another address of that lane.  No instruction.
+static __device__ __forceinline__ void eas_wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // threadIdx.x as a value of its own: the address arithmetic of the bodies sharing an entry is not
 // merged and kept in registers across their branches (with it merged, the entry spilled)
 static __device__ __forceinline__ int eas_tid() {
@@ -1030,7 +1038,7 @@ static __device__ __forceinline__ void eas_gemm_skinny_dma(const eas_op_t* __res
 // Skinny path for inputs the DMA cannot take (f32, odd K, odd ldb, odd addresses): 64 columns
 // from n0, the four waves split K as above, each moving its range global -> registers -> LDS, R
 // stages of 32 k in flight in registers.  A wave's LDS accesses run in order, so its private slot
-// needs no barrier.  Bound by the rows of B from HBM where the grid fills the chip, else by the latency of
+// needs no barrier (only the compiler has to keep that order: eas_wave_order).  Bound by the rows of B from HBM where the grid fills the chip, else by the latency of
 // a wave's chain of stages.  With B in the memory-side cache f16 16 x 14336 x 4097 takes 19.6 us, 6.0
 // TB/s, f32 16 x 14336 x 4096 36.1 us, 6.5 TB/s; from HBM 26.4 and 44.2.
 template <typename AT, typename BT, typename CT, int K, int MT>
@@ -1115,10 +1123,12 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
 #pragma unroll
       for (int i = 0; i < NA; ++i) xa[i] = eas_unit_end<AT>(xa[i], lost_a(t, i));
     }
+    eas_wave_order();  // the step before has read the slot
 #pragma unroll
     for (int i = 0; i < NB; ++i) eas_store_unit<BT>(bs + lb[i], xb[i]);
 #pragma unroll
     for (int i = 0; i < NA; ++i) eas_store_unit<AT>(as + la[i], xa[i]);
+    eas_wave_order();
     if (decltype(steady)::value || t + R < nsteps) load(t + R, xa, xb, steady);
     eas_h8 a[MT];
 #pragma unroll
