@@ -303,7 +303,8 @@ class Kernel:
         it.  False: not such a call, nothing done."""
         grid = kwargs["_grid"]
         if type(grid) is not tuple or not kwargs.keys() <= self._grid_kw \
-                or type(kwargs.get("_tptg", ())) is not tuple:
+                or type(kwargs.get("_tptg", ())) is not tuple \
+                or type(kwargs.get("_sync", True)) is not bool:  # 1 == True as a key, but is refused
             return False
         kw = tuple([item for item in kwargs.items() if item[0] != "_grid"])
         try:

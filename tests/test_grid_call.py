@@ -62,6 +62,19 @@ def test_which_calls_take_the_grid_launch(monkeypatch):
             k(a, a, a, 64, BLOCK=64, **bad)
 
 
+@pytest.mark.parametrize("sync", [1, 0, 1.0, None, np.True_])
+def test_a_sync_that_is_no_bool_is_refused_after_one_that_equals_it(monkeypatch, sync):
+    rt = _Runtime()
+    monkeypatch.setattr(eas_kernel, "get_runtime", lambda *a, **k: rt)
+    k = eas.kernel(K.add_kernel.fn)
+    a = np.ones(64, np.float32)
+    for s in (True, False):
+        k(a, a, a, 64, BLOCK=64, _grid=(1, 1), _sync=s)
+    with pytest.raises(TypeError, match="_sync must be bool"):
+        k(a, a, a, 64, BLOCK=64, _grid=(1, 1), _sync=sync)
+    assert len(rt.runs) == 2 and not rt.fast
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("sync", [True, False])
 @pytest.mark.parametrize("kind", ["mma", "tiled"])
