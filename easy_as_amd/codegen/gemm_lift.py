@@ -1199,21 +1199,30 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
     tiles64 = -(-m // 64) * -(-n // 64)
     choice = _gemm_entry_choice()
     if m <= p.get("skinny_m", 0):
-        # The 4-wave entry runs its skinny path for every launch of at most skinny_m rows (one
-        # workgroup per skinny_n columns, all rows), so it is only ever launched on that grid.
-        # Up to WIDE_M rows, a launch whose groups would take more than one round of CUs gets
+        # The 4-wave entry runs its skinny path on one workgroup per skinny_n columns, all rows.  Up
+        # to WIDE_M rows, a launch whose groups would take more than one round of CUs gets
         # twice the columns per workgroup (the kernel reads which from the grid).  From 17 rows
         # on, a launch whose groups still take more than one round goes to the 128 x 128 entry
         # instead (or to the entry EAS_HIP_GEMM_ENTRY names).
         groups = -(-n // p["skinny_n"])
         if m <= WIDE_M and groups > compute_units:
             groups = -(-n // (2 * p["skinny_n"]))
-        # Operands the DMA entries cannot take run 64 x 64 register tiles above 64 rows (128 x 4096 x
-        # 1024 f32 on 64 skinny groups 17.5 us, on 128 tiles 7.8; 100 x 4097 x 1023 f16 15.0 and 8.9).
+        # Above 64 rows only operands its DMA takes (16-byte aligned rows) run the skinny path.  Rows at
+        # 4 bytes go to the smallest of the DMA entries' tiles of 64 x 64, 128 x 64 and 128 x 128 that takes
+        # one round of CUs (us on the skinny path's register body and on each: 100 x 4098 x 1022 f16 13.6,
+        # 8.7, 9.8, 12.1; 128 x 8194 x 1022 15.1, 14.5, 11.5, 12.9; 128 x 16390 x 1000 27.4, 23.0, 21.2,
+        # 15.1), any others to 64 x 64 register tiles (128 x 4096 x 1024 f32 on 64 skinny groups 17.5, on
+        # 128 tiles 7.8; 100 x 4097 x 1023 f16 15.0 and 8.9).
         other = None
         fits = p.get("pp_entry") and _dma_fits(p, runtime_args, K, ldb, m, n_lo, n)
-        if m > 64 and not fits:
+        skinny = m <= 64 or (fits and _rows_at(p, runtime_args, K, ldb, n_lo, 16))
+        if not skinny and (not fits or choice == "4wave" or
+                           (choice == "auto" and not _rows_at(p, runtime_args, K, ldb, n_lo, 4))):
             other = LaunchPlan((tiles64, 1, 1), (p["threads"], 1, 1), hidden)
+        elif not skinny and choice == "auto":
+            t, entry = (tiles64, p["t64_entry"]) if tiles64 <= compute_units else \
+                (tiles128x64, p["t128x64_entry"]) if tiles128x64 <= compute_units else (tiles128, p["t128_entry"])
+            other = LaunchPlan((t, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=entry)
         elif m > SKINNY_CUT and fits:
             if choice == "tile128" or (choice == "auto" and groups > compute_units):
                 other = LaunchPlan((tiles128, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t128_entry"])
@@ -1308,3 +1317,26 @@ def _dma_fits(p: dict, runtime_args: Any, K: int, ldb: int, m: int, n_lo: int, n
         if callable(ptr) and int(ptr()) % 4:
             return False
     return True
+
+
+def _rows_at(p: dict, runtime_args: Any, K: int, ldb: int, n_lo: int, nbytes: int) -> bool:
+    """Whether the rows of 16-bit A and B start at multiples of ``nbytes``, after the move to the
+    rectangle's origin: the operands' addresses are known for torch tensors and GPU ``eas.Tensor``s, and
+    NumPy inputs are staged into allocations of their own."""
+    step = nbytes // 2
+    if K % step or ldb % step or n_lo % step:
+        return False
+    return all(_address(runtime_args.get(name)) % nbytes == 0 for name in (p["a"], p["b"]))
+
+
+def _address(v: Any) -> int:
+    """Device address of a buffer argument, 0 where it has none yet."""
+    ptr = getattr(v, "data_ptr", None)
+    if callable(ptr):
+        return int(ptr())
+    hip = getattr(v, "_hip", None)  # a GPU eas.Tensor's storage
+    if hip is None:
+        return 0
+    from ..runtime.hip_ext import load_hip_ext
+
+    return int(load_hip_ext(require=True).buffer_info(hip.buf)[0])

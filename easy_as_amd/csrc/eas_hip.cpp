@@ -678,6 +678,11 @@ bool dma_fits(uint64_t a_ptr, uint64_t b_ptr, uint64_t K, uint64_t ldb, uint64_t
   return a_ptr % 4 == 0 && b_ptr % 4 == 0;
 }
 
+// Whether the rows of 16-bit A and B start at 16-byte boundaries, as the skinny path's DMA wants them.
+bool rows_at_16(uint64_t a_ptr, uint64_t b_ptr, uint64_t K, uint64_t ldb, uint64_t n_lo) {
+  return K % 8 == 0 && ldb % 8 == 0 && n_lo % 8 == 0 && a_ptr % 16 == 0 && b_ptr % 16 == 0;
+}
+
 uint64_t cdiv(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
 // Workgroups of the main entry's register body (operands the DMA cannot take): the tile with the
@@ -780,18 +785,24 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g
     threads = t;
   };
   if (m <= g->skinny_m) {
-    // The 4-wave entry runs its skinny path for every launch of at most skinny_m rows (one
-    // workgroup per skinny_n columns, all rows), so it is only ever launched on that grid.  Up to
+    // The 4-wave entry runs its skinny path on one workgroup per skinny_n columns, all rows.  Up to
     // wide_m rows, a launch whose groups would take more than one round of CUs gets twice the
     // columns per workgroup (the kernel reads which from the grid).  Above skinny_cut rows, a
     // launch whose groups still take more than one round goes to the 128 x 128 entry instead.
     uint64_t grp = cdiv(n, g->skinny_n);
     if (m <= g->wide_m && grp > cus) grp = cdiv(n, 2ull * g->skinny_n);
     pick(EAS_HIP_GEMM_MAIN, grp, g->threads);
-    // Operands the DMA entries cannot take run 64 x 64 register tiles above 64 rows.
+    // Above 64 rows only operands its DMA takes (16-byte aligned rows) run the skinny path.  Rows at 4
+    // bytes go to the smallest tile of the DMA entries that takes one round of CUs, any others to
+    // 64 x 64 register tiles (plan_gemm holds the measurements).
     const bool dma = has(EAS_HIP_GEMM_PP) && fits();
-    if (m > 64 && !dma) {
+    const bool skinny = m <= 64 || (dma && rows_at_16(a_ptr, b_ptr, g->K, ldb, (uint64_t)n_lo));
+    if (!skinny && (!dma || ch == k4Wave)) {
       wgs = tiles64;
+    } else if (!skinny && ch == kAuto) {
+      if (tiles64 <= cus) pick(EAS_HIP_GEMM_T64X64, tiles64, g->t128_threads);
+      else if (tiles128x64 <= cus) pick(EAS_HIP_GEMM_T128X64, tiles128x64, g->t128_threads);
+      else pick(EAS_HIP_GEMM_T128, tiles128, g->t128_threads);
     } else if (m > g->skinny_cut && dma) {
       if (ch == kTile128 || (ch == kAuto && grp > cus)) pick(EAS_HIP_GEMM_T128, tiles128, g->t128_threads);
       else if (ch == kTile128x256) pick(EAS_HIP_GEMM_T128X256, tiles128x256, g->t128_threads);
