@@ -1056,7 +1056,7 @@ static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict
   constexpr int UA = eas_unit<AT>(), UB = eas_unit<BT>();
   constexpr int ACH = KS / UA, BCH = NT / UB;                  // units per row of A (within a stage) and of B
   constexpr int NA = MR * ACH / 64, NB = KS * BCH / 64;        // units per lane and stage
-  constexpr int R = MT == 8 ? 1 : 2;                           // stages in flight
+  constexpr int R = 2;                                         // stages in flight
   constexpr int STH = KS * NT + MR * KS;                       // halves: B [32][64], A [MR][32]
   const int tid = eas_tid(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1457,14 +1457,14 @@ extern "C" __global__ __launch_bounds__(256) void @NAME@(
   const BT* __restrict__ B = @B@ + __eas_n_lo;
   CT* __restrict__ C = @C@ + (size_t)__eas_m_lo * ldb + __eas_n_lo;
   const int M = (int)(__eas_m_hi - __eas_m_lo), N = (int)(__eas_n_hi - __eas_n_lo);
-  // one LDS array for all bodies: DMA ring 4 x 2 x 16 KB, register body 2 x 2 x 256 x 72 halves,
-  // skinny path 4 waves x 4 stages x (4 + MT) KB (3 stages x 12 KB for 8 row tiles)
-  __shared__ __attribute__((aligned(1024))) eas_op_t smem[2 * 2 * 256 * 72];
+  // one LDS array for all bodies, 144 KB: the skinny path's rings, 4 waves x 3 stages x 12 KB at most; the DMA
+  // ring takes 4 x 2 x 16 KB, the register tiles up to 64 KB
+  __shared__ __attribute__((aligned(1024))) eas_op_t smem[147456 / 2];
   // DMA loads take any 4-byte aligned rows (16-byte chunks may straddle alignment and the buffer range,
   // which is checked per dword); the skinny path also wants whole 16-byte chunks per row of A
   const bool dma_ok = OP_IN && (K % 2 == 0) && (ldb % 2 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 4 == 0) &&
                       ((uint64_t)M * K * 2 < (1ull << 31)) && (((uint64_t)(K - 1) * ldb + N) * 2 < (1ull << 31));
-  const bool skinny_dma_ok = dma_ok && (K % 8 == 0) && (ldb % 8 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 16 == 0);
+  const bool skinny_dma_ok = dma_ok && (ldb % 8 == 0) && ((((uint64_t)A) | ((uint64_t)B)) % 16 == 0);
   // The grid says which tile the launch plan picked: the smallest whose count it is (where two tiles
   // have the same count either covers C).  256 x 256 also for operands the DMA takes, on its 4-wave body.
   auto count = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -1474,7 +1474,7 @@ extern "C" __global__ __launch_bounds__(256) void @NAME@(
     // one round of CUs; the grid says which.  1, 2, 4 or 8 row tiles of 16.
     const bool wide = wgs * 64 < N;
     const int n0 = (int)blockIdx.x * (wide ? 128 : 64);
-    if constexpr (OP_IN) {
+    if constexpr (OP_IN && K % 8 == 0) {
       if (skinny_dma_ok) {
         const eas_op_t* __restrict__ Ah = (const eas_op_t*)A;
         const eas_op_t* __restrict__ Bh = (const eas_op_t*)B;
@@ -1494,15 +1494,16 @@ extern "C" __global__ __launch_bounds__(256) void @NAME@(
       }
     }
     // inputs the DMA cannot take (on a 128-column grid, 64 columns at a time)
-    if (K < 8 || ldb < 8) {  // rows shorter than a 16-byte unit of 16-bit elements
+    // rows shorter than a 16-byte unit of 16-bit elements; above 64 rows only a guard: the plan sends
+    // operands the DMA cannot take to tiles
+    if (K < 8 || ldb < 8 || M > 64) {
       eas_gemm_elementwise<AT, BT, CT, K, SKINNY_M, 128>(A, B, C, ldb, M, min(N, n0 + (wide ? 128 : 64)), 0, n0);
       return;
     }
     for (int c0 = n0; c0 < min(N, n0 + (wide ? 128 : 64)); c0 += 64) {
       if (M <= 16) eas_gemm_skinny_regs<AT, BT, CT, K, 1>(A, B, C, ldb, M, N, c0, smem);
       else if (M <= 32) eas_gemm_skinny_regs<AT, BT, CT, K, 2>(A, B, C, ldb, M, N, c0, smem);
-      else if (M <= 64) eas_gemm_skinny_regs<AT, BT, CT, K, 4>(A, B, C, ldb, M, N, c0, smem);
-      else eas_gemm_skinny_regs<AT, BT, CT, K, 8>(A, B, C, ldb, M, N, c0, smem);
+      else eas_gemm_skinny_regs<AT, BT, CT, K, 4>(A, B, C, ldb, M, N, c0, smem);
     }
     return;
   }

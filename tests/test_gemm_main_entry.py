@@ -30,3 +30,10 @@ def test_few_row_bodies_have_no_checks_that_always_pass(tmp_path):
     asm = subprocess.run([str(OBJDUMP), "-d", "--mcpu=gfx950", str(path)], check=True, capture_output=True, text=True).stdout
     main = re.search(r"<matmul_mma_kernel>:\n(.*?)\n\n", asm, re.S).group(1)
     assert len(re.findall(r"\tv_cmpx?_", main)) < 1000
+
+
+@pytest.mark.parametrize("k,dtype,limit", [(1023, np.float16, 105_000), (2048, np.float32, 120_000), (1022, np.float16, 190_000)])
+def test_no_bodies_that_no_launch_reaches(k, dtype, limit):
+    # with the few-row DMA body for K off a multiple of 8 and the register body for 65-128 rows:
+    # 110, 127 and 193 KB; without 96, 109 and 179
+    assert len(_code(k, dtype)) < limit

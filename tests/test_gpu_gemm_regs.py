@@ -98,3 +98,10 @@ def test_few_rows_and_short_rows(gpu_runtime, mnk, dtype):
 @pytest.mark.parametrize("mnk,dtype", [((140, 96, 65), "f16"), ((20, 64, 70), "f32"), ((300, 160, 64), "f32")])
 def test_a_rectangle_that_ends_inside_its_rows(gpu_runtime, mnk, dtype):
     _run(gpu_runtime, *mnk, dtype, pad=3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk,dtype", [((100, 129, 65), "f16"), ((65, 200, 72), "f32"), ((128, 130, 48), "bf16")])
+def test_guard_of_a_few_row_grid_above_64_rows(gpu_runtime, mnk, dtype):
+    # one workgroup per 64 columns for operands the DMA cannot take: the plan launches tiles instead
+    _run(gpu_runtime, *mnk, dtype, grid=K.cdiv(mnk[1], 64), pad=mnk[1] == 130)
