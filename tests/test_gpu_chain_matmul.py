@@ -136,3 +136,17 @@ def test_native_launches_and_a_thread_count(gpu_runtime):
         assert np.array_equal(got[:rows].view(np.uint32), want[:rows].view(np.uint32))
     # the last thread of the last row's threadgroups was left out
     assert np.isnan(got[m - 1, 63]) and np.array_equal(got[m - 1, :63], want[m - 1, :63])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(130, 131, 257), (70, 300, 259), (129, 257, 290), (200, 70, 287), (65, 129, 319)])
+@pytest.mark.parametrize("values", ["normal", "tiny", "special"])
+def test_bit_exact_on_128_tiles_with_a_k_tail(gpu_runtime, monkeypatch, mnk, values):
+    """K off a multiple of 4: the chunk of A that straddles K, with 9 and with 10 stages."""
+    m, n, k = mnk
+    f = np.zeros(8, np.float32)
+    ck = K.matmul_kernel.compile(f, f, f, m, n, BLOCK=64, K=k)
+    monkeypatch.setenv("EAS_HIP_GEMM_ENTRY", "tile128")
+    plan = plan_launch(ck, {"M": m, "N": n}, grid=(m, K.cdiv(n, 64), 1))
+    assert plan.entry == "matmul_kernel__mm__t128" and plan.grid == (K.cdiv(m, 128) * K.cdiv(n, 128), 1, 1)
+    test_bit_exact(gpu_runtime, monkeypatch, mnk, "tile128", values)

@@ -105,3 +105,14 @@ def test_a_rectangle_that_ends_inside_its_rows(gpu_runtime, mnk, dtype):
 def test_guard_of_a_few_row_grid_above_64_rows(gpu_runtime, mnk, dtype):
     # one workgroup per 64 columns for operands the DMA cannot take: the plan launches tiles instead
     _run(gpu_runtime, *mnk, dtype, grid=K.cdiv(mnk[1], 64), pad=mnk[1] == 130)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk,dtype", [((29, 130, 1023), "f16"), ((55, 200, 1000), "f32"), ((40, 131, 771), "bf16"),
+                                       ((9, 129, 1541), "bf16"), ((14, 96, 776), "f32"), ((61, 67, 1031), "f16"),
+                                       ((20, 72, 1030), "f16"),
+                                       # over 256 groups of 64 columns: two of them, in turn, on the same LDS
+                                       ((20, 16451, 771), "f16"), ((50, 16450, 1000), "f32"), ((7, 16391, 1023), "bf16")])
+def test_few_rows_steady_loop(gpu_runtime, mnk, dtype):
+    # K above 512: each of the four waves has more than the 4 stages of 32 k that the loop without a branch needs
+    _run(gpu_runtime, *mnk, dtype)
