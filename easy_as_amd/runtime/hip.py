@@ -386,15 +386,13 @@ class HipRuntime:
 
     def grid_launcher(self, ck: Any, names: tuple[str, ...], args: tuple[Any, ...], sync: bool) -> Any:
         """``fast_launcher`` for launches whose ``_grid`` is a tuple of ints: the returned callable
-        takes the call's arguments and its grid.  Every kernel kind, a lifted GEMM (whose plan the
-        native layer makes from its arguments on each call) with torch tensors only."""
+        takes the call's arguments and its grid.  Every kernel kind; a lifted GEMM's plan the
+        native layer makes from its arguments on each call."""
         geo = ck.geometry
         if geo is None or geo.kind not in ("spmd", "thread", "gemm"):
             return None
         specs = self._fast_specs(ck, names, args)
-        if specs is None or (geo.kind == "gemm" and any(kind == 4 for kind, _ in specs)):
-            return None
-        return self._fast_launch(ck, specs, -1, sync)
+        return None if specs is None else self._fast_launch(ck, specs, -1, sync)
 
     def _fast_specs(self, ck: Any, names: tuple[str, ...], args: tuple[Any, ...]) -> list[tuple[int, Any]] | None:
         """Per-argument (kind, expected dtype or type) of a native fast launch, None when an

@@ -62,6 +62,43 @@ def test_which_calls_take_the_grid_launch(monkeypatch):
             k(a, a, a, 64, BLOCK=64, **bad)
 
 
+def test_one_launch_per_kind_of_arguments(monkeypatch):
+    """A launch takes the types it was made for; each kind of arguments keeps its own, or that there is none."""
+    class Typed(_Runtime):
+        def grid_launcher(self, ck, names, args, sync):
+            self.made += 1
+            if args[0].dtype == np.float16:
+                return None
+            launch = super().grid_launcher(ck, names, args, sync)
+            self.made -= 1
+            kind = type(args[0])
+            return lambda call_args, grid: launch(call_args, grid) if type(call_args[0]) is kind else NotImplemented
+
+    rt = Typed()
+    monkeypatch.setattr(eas_kernel, "get_runtime", lambda *a, **k: rt)
+    k = eas.kernel(K.add_kernel.fn)
+    a, h = np.ones(64, np.float32), np.ones(64, np.float16)
+    t = eas.tensor(a, device="cpu")
+
+    def call(x, **kw):
+        k(x, x, x, 64, BLOCK=64, _grid=(1, 1), **kw)
+
+    for x in (a, t, h):
+        call(x)
+    assert len(rt.runs) == 3 and rt.made == 3 and not rt.fast
+    for x in (a, t, a, t, t):  # in turn: never the full path
+        call(x)
+    assert len(rt.runs) == 3 and rt.made == 3 and len(rt.fast) == 5
+    for _ in range(3):  # no launch for this kind: the full path, and none is made anew
+        call(h)
+    assert len(rt.runs) == 6 and rt.made == 3 and len(rt.fast) == 5
+    k(a, a, a, np.uint32(64), BLOCK=64, _grid=(1, 1))  # a scalar of a type no launch takes
+    assert len(rt.runs) == 7 and rt.made == 3
+    for i in range(200):  # bounded
+        k(a, a, a, 64, BLOCK=64, _grid=(1, 1), _tptg=(1,) + (1,) * (i % 3), _sync=bool(i % 2))
+    assert len(k._grid_made) <= 64 and len(k._grid_fast) <= 64
+
+
 @pytest.mark.parametrize("sync", [1, 0, 1.0, None, np.True_])
 def test_a_sync_that_is_no_bool_is_refused_after_one_that_equals_it(monkeypatch, sync):
     rt = _Runtime()
@@ -125,6 +162,41 @@ def test_lifted_matmuls(gpu_runtime, monkeypatch, kind, sync):
     call(96, 64, a, b, c, grid=(0, 2))  # nothing to run
     call(96, 64, a, b, c, grid=(2.0, 3.0))  # as the full path converts it
     check(96, 64, a, b, c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sync", [True, False])
+def test_kinds_of_arguments_in_turn(gpu_runtime, monkeypatch, sync):
+    """f16 and f32 torch tensors and GPU eas.Tensors through one matmul: each on its own specialisation and buffers."""
+    import torch
+
+    mma = eas.kernel(K.matmul_mma_kernel.fn)
+    k = 72
+    g = torch.Generator(device="cuda").manual_seed(1)
+
+    def one(kind, m, n):
+        dt = torch.float32 if kind == "f32" else torch.float16
+        a, b = (torch.empty(s, device="cuda").uniform_(-1, 1, generator=g).half().to(dt) for s in (m * k, k * n))
+        c = torch.full((m * n,), float("nan"), device="cuda")
+        args = [eas.tensor(x, device="hip") for x in (a, b, c)] if kind == "eas" else [a, b, c]
+        torch.cuda.synchronize()  # eas.Tensors alone go on the default stream
+        mma(*args, m, n, BM=32, BN=32, BK=8, K=k, NT=512, _grid=(K.cdiv(n, 32), K.cdiv(m, 32)), _sync=sync)
+        gpu_runtime.synchronize()
+        torch.cuda.synchronize()
+        want = a.view(m, k).double().cpu().numpy() @ b.view(k, n).double().cpu().numpy()
+        assert ops.rel_err(c.view(m, n).cpu().numpy().astype(np.float64), want) <= 1e-5 * k ** 0.5
+
+    for kind in ("f16", "f32", "eas"):
+        one(kind, 200, 136)
+    monkeypatch.setattr(gpu_runtime, "run", lambda *x, **y: (_ for _ in ()).throw(AssertionError("the full path ran")))
+    for kind in ("f32", "eas", "f16", "f32", "f16", "eas"):
+        one(kind, 200, 136)
+        one(kind, 33, 101)
+    monkeypatch.undo()
+    short = eas.tensor(torch.zeros(8, device="cuda", dtype=torch.float16), device="hip")
+    with pytest.raises(ValueError, match="holds"):  # refused before a launch, by the buffer's length
+        mma(short, short, eas.tensor(torch.zeros(8, device="cuda"), device="hip"), 64, 64,
+            BM=32, BN=32, BK=8, K=k, NT=512, _grid=(2, 2), _sync=sync)
 
 
 @pytest.mark.gpu
