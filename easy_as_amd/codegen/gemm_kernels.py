@@ -2171,5 +2171,5 @@ def emit_gemm(ir: IRModule, block: int, spec: GemmSpec, name: str | None = None)
         "t128x64_entry": f"{name}__t128x64" if pingpong else None,
         "t64_entry": f"{name}__t64x64" if pingpong else None,
         "a": spec.a, "b": spec.b, "c": spec.c, "out_dtype": spec.c_dtype.value,
-        "op_dtype": "f32" if spec.f32 else spec.op_dtype.value})
+        "op_dtype": "f32" if spec.f32 else spec.op_dtype.value, "ordered": spec.ordered})
     return Lowered(PRELUDE + header + src, block, "thread", geo)

@@ -1192,12 +1192,14 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
             raise ValueError(f"buffer {name!r} holds {have} elements; this launch touches {n_need}")
     hidden = (m_lo, m_hi, n_lo, n_hi)
     m, n = m_hi - m_lo, n_hi - n_lo
+    choice = _gemm_entry_choice()
+    if p.get("ordered") and choice == "auto" and threads_ahead(K, m, n, ldb, p["TN"]):
+        raise ValueError("the kernel's own threads are the faster")
     tiles = -(-m // p["BM"]) * -(-n // p["BN"])
     tiles128 = -(-m // 128) * -(-n // 128)
     tiles128x256 = -(-m // 128) * -(-n // 256)
     tiles128x64 = -(-m // 128) * -(-n // 64)
     tiles64 = -(-m // 64) * -(-n // 64)
-    choice = _gemm_entry_choice()
     if m <= p.get("skinny_m", 0):
         # The 4-wave entry runs its skinny path on one workgroup per skinny_n columns, all rows.  Up
         # to WIDE_M rows, a launch whose groups would take more than one round of CUs gets
@@ -1283,6 +1285,18 @@ def _register_tiles(m: int, n: int, cus: int) -> int:
         if best is None or cost <= best[0]:
             best = (cost, t)
     return best[1]
+
+
+def threads_ahead(K: int, m: int, n: int, ldb: int, block: int) -> bool:
+    """Whether a launch of the one-thread-per-output matmul is faster on its own threads than on the ordered
+    GEMM.  Rows of B of under 4 columns, which the GEMM's DMA cannot take: 1000 x 1 x 512 29.9 us on threads
+    and 105.7, 4096 x 3 x 130 11.1 and 31.2 (20000 x 3 x 512 158.6 and 139.3).  A short K on a small output,
+    since the GEMM's workgroup fills LDS and runs a whole stage of MFMAs however short K is.  Kernel times in us,
+    threads and GEMM: 32 x 32 x 8 2.1 and 2.8, 64 x 964 x 30 2.6 and 4.1, 500 x 300 x 48 3.6 and 4.6, 1088 x
+    242 x 48 (279 k threads) 4.5 and 4.7; past it 300 x 1000 x 46 (307 k) 5.1 and 4.7, 1000 x 700 x 8 4.6
+    and 4.2, 500 x 300 x 57 5.0 and 4.7, 32 x 32 x 64 7.4 and 3.6.  The same bits
+    either way.  K below 8 (2.0 and 3.0 at 5) is left on the GEMM, where the launch tests have it."""
+    return ldb < 4 or (8 <= K <= 48 and m * -(-n // block) * block <= 288 << 10)
 
 
 _ENTRY_CHOICES = ("auto", "8wave", "tile128", "tile128x256", "tile128x64", "tile64", "4wave")

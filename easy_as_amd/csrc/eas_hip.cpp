@@ -770,6 +770,11 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* s, const eas_hip_gemm_shape* g
                   b.arg, (unsigned long long)have, (unsigned long long)b.need);
   }
   const uint64_t m = (uint64_t)(m_hi - m_lo), n = (uint64_t)(n_hi - n_lo), cus = (uint64_t)compute_units;
+  // rows of B of under 4 columns, or a short K on a small output: the kernel's own threads
+  // (gemm_lift.threads_ahead holds the measurements)
+  if (s->kind == EAS_HIP_KIND_THREAD && ch == kAuto &&
+      (ldb < 4 || (g->K >= 8 && g->K <= 48 && (u128)m * cdiv(n, g->tn) * g->tn <= (288u << 10))))
+    return fail(EAS_HIP_ERR_INVALID, "the kernel's own threads are the faster");
   const uint64_t tiles = cdiv(m, g->bm) * cdiv(n, g->bn), tiles128 = cdiv(m, 128) * cdiv(n, 128);
   const uint64_t tiles128x256 = cdiv(m, 128) * cdiv(n, 256), tiles128x64 = cdiv(m, 128) * cdiv(n, 64);
   const uint64_t tiles64 = cdiv(m, 64) * cdiv(n, 64);

@@ -139,6 +139,20 @@ def test_native_launches_and_a_thread_count(gpu_runtime):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(65, 64, 31), (130, 131, 32), (64, 63, 33), (37, 130, 46), (129, 70, 9)])
+@pytest.mark.parametrize("values", ["normal", "tiny", "special"])
+def test_bit_exact_on_64_tiles_with_a_short_k(gpu_runtime, monkeypatch, mnk, values):
+    """K of 8 to 48 on a small output runs on the kernel's threads unless an entry is named; here the 64 x 64 tiles."""
+    m, n, k = mnk
+    f = np.zeros(8, np.float32)
+    ck = K.matmul_kernel.compile(f, f, f, m, n, BLOCK=64, K=k)
+    assert plan_launch(ck, {"M": m, "N": n}, grid=(m, K.cdiv(n, 64), 1)).entry is None
+    monkeypatch.setenv("EAS_HIP_GEMM_ENTRY", "4wave")
+    assert plan_launch(ck, {"M": m, "N": n}, grid=(m, K.cdiv(n, 64), 1)).entry == "matmul_kernel__mm"
+    test_bit_exact(gpu_runtime, monkeypatch, mnk, "4wave", values)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mnk", [(130, 131, 257), (70, 300, 259), (129, 257, 290), (200, 70, 287), (65, 129, 319)])
 @pytest.mark.parametrize("values", ["normal", "tiny", "special"])
 def test_bit_exact_on_128_tiles_with_a_k_tail(gpu_runtime, monkeypatch, mnk, values):
