@@ -17,9 +17,9 @@ entry points, and the launch plan (``gemm_lift.plan_gemm``) picks one:
   128 x 64 tiles, for launches whose 256 x 256 grid would leave CUs idle: 4 waves
   issue the DMA, 4 waves of 64 x 64 (64 x 128, 32 x 32, 64 x 32) read fragments
   and run the MFMAs.
-* ``<name>`` (256 threads, 4 waves of 128 x 128, 4 x 4 accumulators in 256
-  AGPRs): the skinny path (launches of at most 128 rows), the 4-wave DMA body,
-  and the register body; a uniform branch picks one per launch.
+* ``<name>`` (256 threads): the skinny path (launches of at most 64 rows, and of up to 128
+  whose rows of A and B are 16-byte aligned), the 4-wave DMA body (128 x 128 per wave, 4 x 4
+  accumulators in 256 AGPRs), and the register tiles; a uniform branch picks one per launch.
 
 DMA bodies (A and B of the operand type; K and ldb even and 4-byte aligned bases, so every row
 is 4-byte aligned; each matrix under 2 GiB):
@@ -46,8 +46,9 @@ Register bodies (any other case, including f32 inputs that MFMA consumes as f16)
 global -> registers -> LDS in the DMA bodies' layouts, rounding on the way; 16-byte
 loads at any element alignment, with the ends of rows and buffers moved into place in
 registers.  Launches of at most 64 rows split K over the four waves of a 64-column
-group; others run 64 x 64, 128 x 64, 128 x 128 or 256 x 256 tiles, whichever the launch
-plan's cost rule picks.
+group (also those the skinny path's DMA does not take, rows off 16 bytes); 65-128 rows run 64 x 64
+tiles, others 64 x 64, 128 x 64, 128 x 128 or 256 x 256 ones, whichever the launch plan's cost rule
+picks.
 
 Tile order is XCD aware: workgroup w runs on XCD w % 8, so each XCD gets a
 contiguous range of tiles, grouped 4 tile-rows high for L2 reuse.
@@ -637,9 +638,9 @@ static __device__ __forceinline__ void eas_gemm_pp(const eas_op_t* __restrict__ 
   }
 }
 
-// Guard body of the 8-wave and smaller-tile entries for inputs the DMA cannot take (the launch plan
-// sends those to the 4-wave entry; this path only keeps a mistaken plan correct): one f32 dot
-// product per element of the TM x TN tile.
+// One f32 dot product per element of the TM x TN tile: the main entry's body for rows of under 8
+// elements (K or ldb), and a guard elsewhere: in the 8-wave and smaller-tile entries for operands the
+// plan could not see to be out of the DMA's reach, in the main entry for a few-row grid above 64 rows.
 template <typename AT, typename BT, typename CT, int K, int TM = 256, int TN = TM>
 static __device__ __forceinline__ void eas_gemm_elementwise(const AT* __restrict__ A, const BT* __restrict__ B,
                                                             CT* __restrict__ C, int ldb, int M, int N, int m0, int n0) {
@@ -918,8 +919,8 @@ static __device__ __forceinline__ void eas_gemm_t128(const eas_op_t* __restrict_
   }
 }
 
-// Skinny path (M <= 128, decode-like): one workgroup per NT = 64 columns (128 for launches whose
-// 64-column groups would need more than one round of CUs), the four waves split K.  Each wave
+// Skinny path (M <= 128, decode-like, rows of A and B at 16 bytes): one workgroup per NT = 64 columns (128
+// for launches whose 64-column groups would need more than one round of CUs), the four waves split K.  Each wave
 // streams its K range of B (and A) HBM -> LDS into a private ring of 4 stages (3 or 2 where 4
 // would not fit the LDS; no barriers in the loop), multiplies MT row tiles of 16
 // (1, 2, 4 or 8) by NT / 16 column tiles with v_mfma_f32_16x16x32_f16 (B transposed by
@@ -1049,9 +1050,9 @@ static __device__ __forceinline__ void eas_gemm_skinny_dma(const eas_op_t* __res
 // Skinny path for inputs the DMA cannot take (f32, odd K, odd ldb, odd addresses): 64 columns
 // from n0, the four waves split K as above, each moving its range global -> registers -> LDS, R
 // stages of 32 k in flight in registers.  A wave's LDS accesses run in order, so its private slot
-// needs no barrier (only the compiler has to keep that order: eas_wave_order).  Bound by the rows of B from HBM where the grid fills the chip, else by the latency of
-// a wave's chain of stages.  With B in the memory-side cache f16 16 x 14336 x 4097 takes 19.6 us, 6.0
-// TB/s, f32 16 x 14336 x 4096 36.1 us, 6.5 TB/s; from HBM 26.4 and 44.2.
+// needs no barrier (only the compiler has to keep that order: eas_wave_order).  Bound by the rows of B from
+// HBM where the grid fills the chip, else by the latency of a wave's chain of stages.  With B in the memory-side cache f16 16 x 14336 x 4097 takes 19.3 us, 6.1
+// TB/s, f32 16 x 14336 x 4096 36.4 us, 6.5 TB/s; from HBM 26.8 and 44.6.
 template <typename AT, typename BT, typename CT, int K, int MT>
 static __device__ __forceinline__ void eas_gemm_skinny_regs(const AT* __restrict__ A, const BT* __restrict__ B,
                                                             CT* __restrict__ C, int ldb, int M, int N, int n0,
@@ -1388,7 +1389,10 @@ static __device__ __forceinline__ void eas_gemm_regs(const AT* __restrict__ A, c
   for (int i = 0; i < TI; ++i) read_a(0, 0, i);
   // Four stages an iteration (two of f32): slots are immediates of the LDS accesses, and the
   // accumulators the compiler moves once an iteration cost less.  Up to 16 stages of 16-bit operands
-  // no loop at all (1531 x 2047 x 1023 f16 16.3 us, 17.1 with it).  256 x 256 has no registers for any.
+  // no loop at all: 1531 x 2047 on 128 x 128 tiles, f16, us without and with it: K = 1023 17.0 and 17.6, 767
+  // 14.8 and 15.5, 511 12.2 and 12.4, 255 level; 700 x 1501 on 128 x 64 level.  Beyond, the code of each
+  // new K would grow for less: K = 1279 19.6 and 20.2, 1535 22.2 and 23.0 (107 KB against 90), 2047 27.3
+  // and 28.3 (118 KB).  256 x 256 has no registers for any.
   constexpr bool BITS16 = sizeof(AT) == 2 && sizeof(BT) == 2;
   constexpr int STEADY = KT > 3 ? KT - 3 : 0, FOURS = BM == 256 || !BITS16 ? 0 : STEADY / 4 * 4;
   constexpr int PAIRS = BM == 256 ? 0 : STEADY / 2 * 2, FLAT = KT <= 16 && BITS16 && BM != 256 ? 4 : 1;
@@ -2098,7 +2102,7 @@ THREADS = 256
 PP_THREADS = 512  # the 8-wave (ping-pong) entry of f16 GEMMs
 T128_THREADS = 512  # the smaller-tile entries of f16 GEMMs: 4 consumer + 4 producer waves
 F32_THREADS = 512  # both fp32 entries: 4 consumer + 4 producer waves
-SKINNY_M = 128  # launches of at most this many rows run the skinny path: one workgroup per SKINNY_N columns
+SKINNY_M = 128  # most rows of the skinny path: one workgroup per SKINNY_N columns
 SKINNY_N = 64
 # MFMA shape of the 8-wave and smaller-tile entries' bodies: 16 (v_mfma_f32_16x16x32, the default) or
 # 32 (v_mfma_f32_32x32x16).  Measured on MI355X with random inputs, where the part runs

@@ -8,7 +8,7 @@ only then, replaces it with hand-written MFMA kernels (``codegen/gemm_kernels.py
 ``v_mfma_f32_16x16x32_f16`` (or ``_bf16``) by default, A and B moved HBM -> LDS by
 ``buffer_load ... lds`` DMA rings in their row-major layouts, B transposed on its
 way out of LDS by ``ds_read_b64_tr_b16``; operands the DMA cannot take (f32
-inputs, rows not 4-byte aligned) run a register-staged body instead.  The fp32
+inputs, rows not 4-byte aligned) run bodies that load through registers instead.  The fp32
 tiled ``dot`` pattern lifts to ``v_mfma_f32_32x32x2_f32`` the same way.
 
 Proof method (no pattern matching on source text): the IR is executed
@@ -1214,7 +1214,9 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
         # one round of CUs (us on the skinny path's register body and on each: 100 x 4098 x 1022 f16 13.6,
         # 8.7, 9.8, 12.1; 128 x 8194 x 1022 15.1, 14.5, 11.5, 12.9; 128 x 16390 x 1000 27.4, 23.0, 21.2,
         # 15.1), any others to 64 x 64 register tiles (128 x 4096 x 1024 f32 on 64 skinny groups 17.5, on
-        # 128 tiles 7.8; 100 x 4097 x 1023 f16 15.0 and 8.9).
+        # 128 tiles 7.8; 100 x 4097 x 1023 f16 15.0 and 8.9).  16-bit results are as exact as on four
+        # waves' part sums (2.08e-4 f16, 1.66e-3 bf16 at K = 1022 and 4094); f32 ones are one chain of sums,
+        # as in every launch of more rows (2.0e-7 against 1.1e-7 at K = 1022, 4.1e-7 and 2.1e-7 at 4094).
         other = None
         fits = p.get("pp_entry") and _dma_fits(p, runtime_args, K, ldb, m, n_lo, n)
         skinny = m <= 64 or (fits and _rows_at(p, runtime_args, K, ldb, n_lo, 16))
@@ -1251,7 +1253,9 @@ def plan_gemm(geo: Any, groups: tuple[int, int, int], runtime_args: Any, live_x:
         # If even 128 x 128 would fill at most half of the CUs: 64 x 64 tiles while they take one round
         # of CUs, else 128 x 64 (twice the 128 x 128 count: one round): us on 128 x 64 and 64 x 64,
         # 1280^3 10.5 and 11.8 (1.56 rounds), 1792 x 1024 x 4096 23.4 and 30.3 (1.75), 1280 x 1280 x
-        # 512 6.5 and 7.1.  Up to 256 k a call is its launch (5.5 and 5.7) and 64 x 64 may take 1.75.
+        # 512 6.5 and 7.1.  Up to 256 k 64 x 64 may take 1.75 rounds, which is a matter of 0.2 us either
+        # way (kernel times at 1280 x 1280 x 64 5.1 and 5.1, x 128 5.4 and 5.3, x 192 5.6 and 5.7, x 256
+        # 5.8 and 6.0).
         small = choice == "auto" and 2 * tiles <= compute_units
         if choice == "tile128x256" or (small and tiles128 > compute_units):
             return LaunchPlan((tiles128x256, 1, 1), (p["t128_threads"], 1, 1), hidden, entry=p["t128x256_entry"])
@@ -1317,9 +1321,10 @@ def _dma_fits(p: dict, runtime_args: Any, K: int, ldb: int, m: int, n_lo: int, n
     """Whether the DMA entries take this launch.  16-bit f16/bf16 (``elem`` 2): every row of A and B
     (after the move to the rectangle's origin) 4-byte aligned; fp32 (``elem`` 4, its 128 x 128 entry):
     rows of B from 4 columns on, K a multiple of 4 or from 256 on (2047^3 120.1 us on 128 x 128 tiles
-    against 127.0 on 64 x 64, 2048 x 2048 x 382 29.0 against 30.3; below, neither is ahead by much:
-    2048 x 2048 x 62 10.9 against 11.6, 4096 x 4096 x 254 78.3 against 75.7, and those stay on 64 x
-    64); each operand's extent under 2 GiB.  Device addresses are known here for torch tensors; numpy
+    against 127.0 on 64 x 64, 2048 x 2048 x 382 29.0 against 30.3; below, neither is ahead throughout
+    and launches stay on 64 x 64: 2048 x 2048 x 46 11.6 against 12.7, x 62 11.8 against 12.6, x 126 16.2
+    against 16.0, x 190 20.1 against 19.8, x 254 24.5 against 23.9, 4096 x 4096 x 254 87.9 against 91.2);
+    each operand's extent under 2 GiB.  Device addresses are known here for torch tensors; numpy
     inputs are staged into fresh allocations, and the entries re-check the addresses they get (a
     misaligned operand takes their slow element-wise guard rather than a wrong result)."""
     if (K % 2 or ldb % 2 or n_lo % 2) if elem == 2 else (ldb < 4 or (K % 4 and K < 256)):

@@ -191,7 +191,7 @@ typedef struct eas_hip_gemm_shape {
   uint32_t row_axis;          /* threadgroup axis (0 or 1) that indexes tile rows                    */
   uint32_t bm, bn;            /* tile of the kernel's own entry                                      */
   uint32_t threads, pp_threads, t128_threads; /* workgroup sizes: own, 8-wave, smaller-tile entries  */
-  uint32_t skinny_m, skinny_n;  /* launches of <= skinny_m rows: one workgroup per skinny_n columns  */
+  uint32_t skinny_m, skinny_n;  /* most rows of the skinny path: one workgroup per skinny_n columns  */
   uint32_t skinny_cut, wide_m;  /* rows that always stay skinny; rows that may take 2 x skinny_n     */
   uint32_t f32;               /* fp32 operands (the tiled `dot` GEMM), else 16-bit                   */
   uint32_t col_masked;        /* columns bounded by N (else by the launched grid only)               */
