@@ -638,9 +638,9 @@ static __device__ __forceinline__ void eas_gemm_pp(const eas_op_t* __restrict__ 
   }
 }
 
-// One f32 dot product per element of the TM x TN tile: the main entry's body for rows of under 8
-// elements (K or ldb), and a guard elsewhere: in the 8-wave and smaller-tile entries for operands the
-// plan could not see to be out of the DMA's reach, in the main entry for a few-row grid above 64 rows.
+// Guard body: one f32 dot product per element of the TM x TN tile.  In the main entry the body for rows of
+// under 8 elements (K or ldb); a guard in the 8-wave and smaller-tile entries, for operands the plan could
+// not see to be out of the DMA's reach, and in the main entry for a few-row grid above 64 rows.
 template <typename AT, typename BT, typename CT, int K, int TM = 256, int TN = TM>
 static __device__ __forceinline__ void eas_gemm_elementwise(const AT* __restrict__ A, const BT* __restrict__ B,
                                                             CT* __restrict__ C, int ldb, int M, int N, int m0, int n0) {
