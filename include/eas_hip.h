@@ -226,7 +226,8 @@ int eas_hip_kernel_set_gemm(eas_hip_kernel* k, const eas_hip_gemm_shape* gemm);
  * the origin is tm * row_base (tn * col_base) when the kernel offsets its threadgroup
  * ids by a scalar, the extent the launched grid, clamped to M (N) when the kernel
  * bounds rows (columns).  A launch that would read or write past a buffer, or whose
- * matrices exceed u32 indexing, is EAS_HIP_ERR_INVALID.  `choice` names the entry
+ * matrices exceed u32 indexing, is EAS_HIP_ERR_INVALID, and with a thread kernel's
+ * shape and "auto" one that its own threads are the faster on.  `choice` names the entry
  * ("auto", "8wave", "tile128", "tile128x256", "tile128x64", "tile64", "4wave");
  * NULL reads EAS_HIP_GEMM_ENTRY (default "auto"). */
 int eas_hip_plan_gemm(const eas_hip_launch_shape* shape, const eas_hip_gemm_shape* gemm, const void* kernarg,
@@ -238,8 +239,8 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* shape, const eas_hip_gemm_shap
  * kernel's own arguments only (shape->arg_bytes when known); the hidden extents are
  * appended here.  `arg_bytes` (nargs entries, one per kernel argument: the byte length
  * of a buffer, 0 for a scalar) stands for the lengths the reference's buffer objects
- * carry; a lifted GEMM needs it to check its extents and rejects NULL, the other kinds
- * ignore it.  Asynchronous.  Replaces `launch` / `launch_async` (_metal.mm:1013-1222,
+ * carry; a lifted GEMM needs it to check its extents and rejects NULL, a thread kernel
+ * with a GEMM beside it takes the GEMM only with it, the other kinds ignore it.  Asynchronous.  Replaces `launch` / `launch_async` (_metal.mm:1013-1222,
  * 1381-1383) and `launch_tg` / `launch_tg_async` (_metal.mm:1232-1379). */
 int eas_hip_launch_threads(const eas_hip_kernel* k, const void* kernarg, size_t kernarg_size,
                            const uint64_t* arg_bytes, int nargs, const uint64_t threads_per_grid[3],
