@@ -240,7 +240,8 @@ int eas_hip_plan_gemm(const eas_hip_launch_shape* shape, const eas_hip_gemm_shap
  * appended here.  `arg_bytes` (nargs entries, one per kernel argument: the byte length
  * of a buffer, 0 for a scalar) stands for the lengths the reference's buffer objects
  * carry; a lifted GEMM needs it to check its extents and rejects NULL, a thread kernel
- * with a GEMM beside it takes the GEMM only with it, the other kinds ignore it.  Asynchronous.  Replaces `launch` / `launch_async` (_metal.mm:1013-1222,
+ * with a GEMM beside it takes the GEMM only with it, the other kinds ignore it.
+ * Asynchronous.  Replaces `launch` / `launch_async` (_metal.mm:1013-1222,
  * 1381-1383) and `launch_tg` / `launch_tg_async` (_metal.mm:1232-1379). */
 int eas_hip_launch_threads(const eas_hip_kernel* k, const void* kernarg, size_t kernarg_size,
                            const uint64_t* arg_bytes, int nargs, const uint64_t threads_per_grid[3],
